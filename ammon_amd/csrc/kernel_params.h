@@ -84,6 +84,7 @@ typedef struct {
    * least warm_min_pos. */
   const void *warm;
   uint32_t warm_row_bytes, warm_rows, warm_bytes, warm_blocks, warm_min_pos;
+  uint32_t tokens;          /* prefill tiles: query tokens of the launch */
 } ammon_k_attention;
 
 typedef struct {

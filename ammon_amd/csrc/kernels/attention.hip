@@ -8,7 +8,7 @@
 // (-amdgpu-kernarg-preload-count): the position load, which every request of
 // the unit waits for, then goes out without a kernel-argument load before it.
 // The parameter struct follows (its copy of the pointer is ignored).
-#include "attention_impl.h"
+#include "attention_prefill_impl.h"
 
 #define ATT_KERNEL(NAME) \
   extern "C" __global__ __launch_bounds__(AMMON_WG) void NAME(const ammon_k_step *step, \
@@ -97,3 +97,34 @@ ATT_KERNEL(ammon_attention_combine_waves) {
   const uint32_t h = blockIdx.x * AMMON_WAVES + (threadIdx.x >> 6);
   if (h < t.q_heads) attention_combine_wave(t, h);
 }
+
+// Prefill tiles: one workgroup per (128 query rows, split, kv head), two per CU
+// (registers and LDS allow two).  Unit u = (tile, split, kv head), kv head
+// fastest, tiles from the last (with causal masking the longest) to the first:
+// with 8 kv heads each XCD keeps one head's K and V in its L2.  Workgroups
+// 0..255 land on distinct CUs; where the rest fit beside them they take their
+// units in reverse, so that a CU that runs two gets a long and a short one.
+#define ATT_PREFILL(NAME, KV, DB, NQ, OCC)                                                   \
+  ATT_KERNEL_OCC(NAME, OCC) {                                                        \
+    ATT_PARAMS(p);                                                                   \
+    __shared__ u32x4 lds[4096];                                                      \
+    const uint32_t rows = p.tokens * (p.q_heads / p.kv_heads);                       \
+    const uint32_t tiles = (rows + PF_ROWS - 1) / PF_ROWS;                           \
+    const uint32_t b = blockIdx.x >> 3, nb = gridDim.x >> 3;                         \
+    const uint32_t u = (b < 32 || nb > 64 ? b : 32 + nb - 1 - b) * 8 + (blockIdx.x & 7u);       \
+    if (u >= tiles * p.splits * p.kv_heads) return; /* uniform */                    \
+    const uint32_t g = u % p.kv_heads, q = u / p.kv_heads;                           \
+    PrefillTile<KV, DB, NQ> unit;                                                       \
+    unit.run(p, g, tiles - 1 - q / p.splits, q % p.splits, (char *)lds);             \
+  }
+ATT_PREFILL(ammon_attention_prefill_f32_d1, float, 1, 1, 2)
+ATT_PREFILL(ammon_attention_prefill_f32_d2, float, 2, 1, 2)
+ATT_PREFILL(ammon_attention_prefill_f32_d3, float, 3, 1, 2)
+ATT_PREFILL(ammon_attention_prefill_f32_d4, float, 4, 1, 2)
+// q whole (three parts), as the VALU units of these shapes take it
+ATT_PREFILL(ammon_attention_prefill_bf16_d1, uint16_t, 1, 3, 2)
+ATT_PREFILL(ammon_attention_prefill_bf16_d2, uint16_t, 2, 3, 2)
+ATT_PREFILL(ammon_attention_prefill_bf16_d3, uint16_t, 3, 3, 2)
+ATT_PREFILL(ammon_attention_prefill_bf16_d4, uint16_t, 4, 3, 1)
+// q as hi + lo, as AttnPartialMfmaStaged takes it (head 128, group a power of two)
+ATT_PREFILL(ammon_attention_prefill_bf16_h128, uint16_t, 4, 2, 2)

@@ -894,21 +894,44 @@ AMMON_DEV void attention_combine_wave(const ammon_k_attention &p, uint32_t h) {
   const float M = wave_max(m);
   const uint32_t d = mine ? 2 * lane : 0;
   float t0 = 0.f, t1 = 0.f, L = 0.f;
-  const uint32_t lanes = min(live, (uint32_t)COMB_SPLIT_LANES);
-  for (uint32_t j = 0; j < lanes; ++j) {
-    float a0 = 0.f, a1 = 0.f, l = 0.f;
-    for (uint32_t s = j; s < live; s += COMB_SPLIT_LANES) {
-      const float *row = base + (size_t)s * slot;
-      const float w = expf(row[head] - M);
-      l = fmaf(row[head + 1], w, l);
-      a0 = fmaf(row[d], w, a0);
-      a1 = fmaf(row[d + 1], w, a1);
+  if (live <= COMB_SPLIT_LANES) {
+    // one split per split lane: eight splits' rows requested at a time (a
+    // row's sum is fmaf(x, w, 0) = x w)
+    for (uint32_t j0 = 0; j0 < live; j0 += 8) {
+      float rm[8], rl[8], r0[8], r1[8];
+#pragma unroll
+      for (uint32_t j = 0; j < 8; ++j) {
+        const float *row = base + (size_t)min(j0 + j, live - 1) * slot;
+        rm[j] = row[head];
+        rl[j] = row[head + 1];
+        r0[j] = row[d];
+        r1[j] = row[d + 1];
+      }
+#pragma unroll
+      for (uint32_t j = 0; j < 8; ++j) {
+        if (j0 + j >= live) break;  // uniform
+        const float w = expf(rm[j] - M);
+        t0 = t0 + fmaf(r0[j], w, 0.f);
+        t1 = t1 + fmaf(r1[j], w, 0.f);
+        L = L + fmaf(rl[j], w, 0.f);
+      }
     }
-    t0 = t0 + a0;
-    t1 = t1 + a1;
-    L = L + l;
+  } else {
+    for (uint32_t j = 0; j < COMB_SPLIT_LANES; ++j) {
+      float a0 = 0.f, a1 = 0.f, l = 0.f;
+      for (uint32_t s = j; s < live; s += COMB_SPLIT_LANES) {
+        const float *row = base + (size_t)s * slot;
+        const float w = expf(row[head] - M);
+        l = fmaf(row[head + 1], w, l);
+        a0 = fmaf(row[d], w, a0);
+        a1 = fmaf(row[d + 1], w, a1);
+      }
+      t0 = t0 + a0;
+      t1 = t1 + a1;
+      L = L + l;
+    }
   }
-  if (lanes < COMB_SPLIT_LANES) {  // the idle split lanes' +0
+  if (live < COMB_SPLIT_LANES) {  // the idle split lanes' +0
     t0 = t0 + 0.f;
     t1 = t1 + 0.f;
     L = L + 0.f;

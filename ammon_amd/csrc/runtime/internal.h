@@ -33,6 +33,10 @@ struct Kernels {
   // matrix cores with K/V staged in an LDS ring of 1 or 2 chunk buffers
   hipFunction_t att_partial_h128_f32[kAttGroups] = {};
   hipFunction_t att_partial_staged[2][kAttGroups] = {};
+  // prefill tiles: [kv dtype][ceil(head / 32) - 1]; bf16, head 128,
+  // power-of-two group: the two-part q of att_partial_staged
+  hipFunction_t att_prefill[2][4] = {};
+  hipFunction_t att_prefill_h128_bf16 = nullptr;
   hipFunction_t att_combine = nullptr;
   hipFunction_t att_combine_waves = nullptr;  // one wave per (token, q head)
   hipFunction_t gemv[2][2][kGemvModes] = {};

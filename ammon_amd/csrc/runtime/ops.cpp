@@ -280,6 +280,59 @@ hipFunction_t attention_kernel(ammon_runtime *rt, ammon_dtype kv_dtype, uint32_t
   return h128 ? rt->k.att_partial_h128_f32[gi] : rt->k.att_partial[dt][ci][gi];
 }
 
+// Prefill attention: query tiles (attention_prefill_impl.h), or decode's units
+// once per token?
+struct PrefillPlan {
+  hipFunction_t f = nullptr;  // NULL: decode's units
+  uint32_t units = 0, split_len = 0, splits = 0;
+};
+
+// Tiles need whole 16-byte pieces of cache rows.  Their splits fill two
+// workgroups per CU and no more, are at least 256 positions (a merge costs as
+// much as three chunks) and at most as many as the caller's scratch holds.
+//
+// A tile's time is its serial chain of chunks whatever the number of rows, a
+// unit's is short but there is one per token, so the two are estimated, in
+// nanoseconds per 64 positions of a tile and per position of a unit.  Measured
+// at 32 q / 8 kv heads of 128 (units, tiles, us): bf16 cache, 32 tokens after
+// 500: 15, 21; 64 after 500: 17, 28; 64 after 4000: 79, 48; 128 after 1000: 71,
+// 32; 300 after 3000: 339, 74.  fp32 cache, 64 after 4000: 163, 146; 128 after
+// 1000: 154, 86; 300 after 3000: 716, 233.
+PrefillPlan prefill_plan(ammon_runtime *rt, uint32_t tokens, uint32_t q_heads, uint32_t kv_heads,
+                         uint32_t head, uint32_t ctx, uint32_t scratch_splits, ammon_dtype kv_dtype,
+                         bool aligned) {
+  PrefillPlan plan;
+  const bool bf = kv_dtype == AMMON_BF16;
+  const uint32_t g = q_heads / kv_heads;
+  const uint64_t rows = (uint64_t)tokens * g, krow = head * dsize(kv_dtype);
+  if (!aligned || krow % 16 != 0 || ctx * krow >= (1ull << 31) || rows >= (1ull << 31)) return plan;
+  const uint64_t units = (uint64_t)cdiv(rows, 128) * kv_heads;
+  const uint64_t slots = 2ull * std::max(rt->info.compute_units, 1);
+  const uint64_t want = std::min<uint64_t>(std::max<uint64_t>(slots / units, 1), scratch_splits);
+  const uint32_t split_len = std::max<uint32_t>(cdiv(cdiv(ctx, want), 64) * 64, 256);
+  const uint32_t splits = cdiv(ctx, split_len);
+  if (units * splits >= (1ull << 31)) return plan;
+  const bool staged = bf && head == 128 && (g & (g - 1)) == 0;
+  const uint32_t db = cdiv(head, 32);
+  const double chunk_ns = staged ? 2200 : bf ? 300 + 780 * db : 2000 + 1800 * db;
+  const double rounds = std::max(1.0, (double)units * splits / slots);
+  const double tile_ns = 9e3 + chunk_ns * cdiv(std::min(split_len, ctx), 64) * rounds +
+                         (splits > 1 ? 8e3 : 0);
+  // a VALU unit's lanes cover the head and its heads the group in powers of two
+  uint32_t lanes = 2, heads = 1;
+  while (lanes < head) lanes <<= 1;
+  while (heads < g) heads <<= 1;
+  const double positions = (double)tokens * kv_heads * (ctx - tokens / 2.0);
+  const double position_ns = staged ? 0.034 : lanes * (head == 128 ? 1.3e-4 * (heads + 1) : 2e-4 * (heads + 0.3));
+  const double unit_ns = 8e3 + positions * position_ns;
+  if (tile_ns >= unit_ns) return plan;
+  plan.f = staged ? rt->k.att_prefill_h128_bf16 : rt->k.att_prefill[bf ? 1 : 0][(head - 1) / 32];
+  plan.units = (uint32_t)units;
+  plan.split_len = split_len;
+  plan.splits = splits;
+  return plan;
+}
+
 ammon_status attention_check(ammon_runtime *rt, const char *what, uint32_t q_heads,
                              uint32_t kv_heads, uint32_t head, uint32_t seq, uint32_t split_len) {
   (void)rt;
@@ -426,7 +479,7 @@ ammon_status attention_pass1(ammon_runtime *rt, ammon_stream stream, const float
   const uint32_t splits = ammon_attention_splits(seq, split_len);
   ammon_k_attention p = {q, k_cache, v_cache, (const ammon_k_step *)step, partial, single_out,
                          q_heads, kv_heads, head, seq, split_len, splits, 0, seq,
-                         single_out ? 1u : 0u, nullptr, 0, 0, 0, 0, 0};
+                         single_out ? 1u : 0u, nullptr, 0, 0, 0, 0, 0, 1};
   return launch_att(rt, stream, f, splits, kv_heads, 1, p, "attention_partial");
 }
 }  // namespace
@@ -479,7 +532,7 @@ ammon_status ammon_attention_combine_warm(ammon_runtime *rt, ammon_stream stream
   VALIDATE_ONLY();
   ammon_k_attention p = {nullptr, nullptr, nullptr, (const ammon_k_step *)step, (float *)partial,
                          out, q_heads, 1, head, seq, split_len,
-                         ammon_attention_splits(seq, split_len), 0, seq, 0, nullptr, 0, 0, 0, 0, 0};
+                         ammon_attention_splits(seq, split_len), 0, seq, 0, nullptr, 0, 0, 0, 0, 0, 1};
   const uint32_t grid = q_heads * cdiv(head, 8);
   if (next_w) {
     // The next GEMV (a RESIDUAL-mode ammon_gemv of next_rows x next_n) gives
@@ -609,9 +662,21 @@ ammon_status ammon_attention_prefill(ammon_runtime *rt, ammon_stream stream, con
   // out-of-range treatment -- NaN output, no partial -- like one past seq
   const uint32_t splits = ammon_attention_splits(ctx, split_len);
   ammon_k_attention p = {q, k_cache, v_cache, (const ammon_k_step *)step, partial, out,
-                         q_heads, kv_heads, head, seq, split_len, splits, 0, ctx, 0, nullptr, 0, 0, 0, 0, 0};
-  st = launch_att(rt, stream, f, splits, kv_heads, tokens, p, "attention_prefill");
-  if (st != AMMON_OK) return st;
+                         q_heads, kv_heads, head, seq, split_len, splits, 0, ctx, 0, nullptr, 0, 0, 0, 0, 0,
+                         tokens};
+  const uintptr_t bits = (uintptr_t)q | (uintptr_t)out | (uintptr_t)k_cache | (uintptr_t)v_cache;
+  const PrefillPlan plan = prefill_plan(rt, tokens, q_heads, kv_heads, head, ctx, splits, kv_dtype,
+                                        (bits & 15u) == 0 && ((uintptr_t)partial & 7u) == 0);
+  if (plan.f) {
+    p.split_len = plan.split_len;
+    p.splits = plan.splits;
+    st = launch_att(rt, stream, plan.f, (plan.units * plan.splits + 7) / 8 * 8, 1, 1, p,
+                    "attention_prefill");
+    if (st != AMMON_OK || p.splits == 1) return st;
+  } else {
+    st = launch_att(rt, stream, f, splits, kv_heads, tokens, p, "attention_prefill");
+    if (st != AMMON_OK) return st;
+  }
   return launch_att(rt, stream, rt->k.att_combine_waves, cdiv(q_heads, kWaves), 1, tokens, p,
                     "attention_prefill");
 }

@@ -122,6 +122,13 @@ static ammon_status load_kernels(ammon_runtime *rt) {
       snprintf(name, sizeof name, "ammon_attention_partial_h128_bf16_lds%d_g%d", 1 << b, gs[g]);
       R(3, name, k.att_partial_staged[b][g]);
     }
+  for (int d = 0; d < 2; ++d)
+    for (int i = 0; i < 4; ++i) {
+      char name[96];
+      snprintf(name, sizeof name, "ammon_attention_prefill_%s_d%d", dtn[d], i + 1);
+      R(3, name, k.att_prefill[d][i]);
+    }
+  R(3, "ammon_attention_prefill_bf16_h128", k.att_prefill_h128_bf16);
   const char *modes[kGemvModes] = {"plain", "residual", "swiglu", "qkv"};
   for (int d = 0; d < 2; ++d)
     for (int v = 0; v < 2; ++v)

@@ -295,6 +295,54 @@ def test_attention_prefill_equals_decode_per_token(rt, q_heads, kv_heads, head, 
         assert rel_err(got[t], want) <= RTOL
 
 
+# The matrix-core tiles (128 query rows x 64 or 32 positions), which long prompts
+# take: heads of one to four 32-dim blocks, whole and ragged; groups that do not
+# divide a tile; last tiles and chunks of a few rows; one split (the scratch stays
+# untouched) and several (start far into the cache).  A token's V that is not
+# finite must reach the tokens from it on and no earlier one, and a position past
+# ctx gives NaN.
+TILE_SHAPES = [  # q_heads, kv_heads, head, kv_dtype, start, tokens, split_len
+    (32, 8, 128, BF16, 0, 333, 1024), (32, 8, 128, BF16, 1100, 130, 64),
+    (16, 16, 128, F32, 0, 900, 1024), (16, 2, 120, BF16, 700, 200, 128),
+    (14, 2, 96, F32, 600, 300, 64), (15, 5, 72, BF16, 0, 500, 512),
+    (32, 8, 64, F32, 1, 511, 1024), (24, 24, 40, BF16, 3, 650, 1024),
+    (32, 32, 24, BF16, 0, 700, 1024), (64, 8, 128, F32, 1000, 65, 256),
+]
+
+
+@pytest.mark.parametrize("q_heads,kv_heads,head,kv_dtype,p0,T,split", TILE_SHAPES)
+def test_attention_prefill_tiles(rt, q_heads, kv_heads, head, kv_dtype, p0, T, split):
+    ctx, late = p0 + T - 2, T // 2  # the last two tokens lie past ctx
+    seq = ctx + 3
+    kc_pm = oracle.storage(oracle.normal(seq * kv_heads * head, 261), kv_dtype).reshape(
+        seq, kv_heads, head)
+    vc_pm = oracle.storage(oracle.normal(seq * kv_heads * head, 262), kv_dtype).reshape(
+        seq, kv_heads, head)
+    qh = oracle.normal(T * q_heads * head, 263).reshape(T, q_heads, head)
+    kc, q = up(rt, head_major(kc_pm, kv_heads, seq, head)), up(rt, qh)
+    nbytes = _abi.lib.ammon_attention_prefill_scratch_bytes(T, q_heads, head, ctx, split)
+    step = rt.step(0, p0)
+    bad_pm = vc_pm.copy()
+    inf = np.inf if kv_dtype == F32 else np.uint16(0x7f80)
+    nan = np.nan if kv_dtype == F32 else np.uint16(0x7fc0)
+    bad_pm[p0 + late, :, 3], bad_pm[p0 + late, :, head - 1] = inf, nan
+    for v_pm, first_bad in ((vc_pm, T - 2), (bad_pm, late)):
+        vc, out = up(rt, head_major(v_pm, kv_heads, seq, head)), rt.alloc(T * q_heads * head * 4)
+        part = up(rt, np.full(nbytes // 4, 7.0, np.float32))
+        call("ammon_attention_prefill", rt.handle, None, q, T, q_heads, kc, vc, kv_dtype, kv_heads,
+             head, seq, step, ctx, split, part, nbytes, out)
+        got = out.download((T, q_heads, head))
+        if split >= ctx:  # one split: a tile writes the result itself
+            np.testing.assert_array_equal(part.download(nbytes // 4), 7.0)
+        for t in (0, 1, 31, 32, late - 1, late, T - 3):
+            if t < first_bad:
+                want = oracle.attention(qh[t], kc_pm, vc_pm, kv_dtype, p0 + t)
+                assert rel_err(got[t], want) <= RTOL, t
+        assert np.isfinite(got[:first_bad]).all()
+        assert np.isnan(got[first_bad:T - 2, :, head - 1]).all()
+        assert np.isnan(got[T - 2:]).all()
+
+
 @pytest.mark.parametrize("kv_dtype", [F32, BF16])
 def test_attention_prefill_positions_past_ctx_are_poisoned(rt, kv_dtype):
     # The grid and the scratch cover ctx positions; the host cannot see
