@@ -48,6 +48,7 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x8 __attribute__((ext_vector_type(8)));
+typedef f32x4 f32x4a4 __attribute__((aligned(4)));  // a 16-byte access at a float's alignment
 
 
 // WQ: 16-byte W loads per lane per step; XQ: LDS quads per lane per (step,
@@ -59,6 +60,51 @@ template <> struct GemmTraits<uint16_t> {
 template <> struct GemmTraits<float> {
   static constexpr int WQ = 2, XQ = 2;
 };
+
+// QKV epilogue of virtual rows (v, v + 1) of token t: rotate q and k pairs
+// with the cos/sin table at position step->position + t; q to y, k and raw
+// v rows to the head-major caches (src/kernels.rs:174-226); a position past
+// the cache poisons q and touches no cache.  fcr, fci: the pair's cos and sin
+// (unused for v rows and positions past the cache).
+AMMON_DEV void qkv_store_pair(const ammon_k_gemm &p, uint32_t t, uint32_t v, float a0, float a1,
+                              float fcr, float fci) {
+#pragma clang fp contract(off)
+  const uint32_t pos = p.step->position + t;
+  const uint32_t kvd = p.kv_dim;
+  if (pos >= p.seq) {
+    if (v < p.d) {
+      p.y[(size_t)t * p.d + v] = __uint_as_float(0x7fc00000u);
+      p.y[(size_t)t * p.d + v + 1] = __uint_as_float(0x7fc00000u);
+    }
+    return;
+  }
+  if (v < p.d + kvd) {
+    const uint32_t rr = v < p.d ? v : v - p.d;
+    const float o0 = a0 * fcr - a1 * fci;
+    const float o1 = a0 * fci + a1 * fcr;
+    if (v < p.d) {
+      p.y[(size_t)t * p.d + v] = o0;
+      p.y[(size_t)t * p.d + v + 1] = o1;
+    } else {
+      store_pair_out(p.k_cache, p.kv_dtype,
+                     ((size_t)(rr / p.head) * p.seq + pos) * p.head + rr % p.head, o0, o1);
+    }
+  } else {
+    const uint32_t rv = v - p.d - kvd;
+    store_pair_out(p.v_cache, p.kv_dtype,
+                   ((size_t)(rv / p.head) * p.seq + pos) * p.head + rv % p.head, a0, a1);
+  }
+}
+
+AMMON_DEV void qkv_store_pair(const ammon_k_gemm &p, uint32_t t, uint32_t v, float a0, float a1) {
+  const uint32_t pos = p.step->position + t, rr = v < p.d ? v : v - p.d;
+  float fcr = 0.f, fci = 0.f;
+  if (pos < p.seq && v < p.d + p.kv_dim) {
+    const float *cs = p.table + (size_t)pos * p.head + rr % p.head;
+    fcr = cs[0], fci = cs[1];
+  }
+  qkv_store_pair(p, t, v, a0, a1, fcr, fci);
+}
 
 // NT 16-token column tiles per workgroup, KC-wide reduction chunks; KS
 // waves share a row tile, each taking every KS-th 32-wide step (KS = 4: one
@@ -229,33 +275,54 @@ struct GemmTile {
   }
 
   // Lane l holds rows 4(l / 16) + r of the wave tile, token tok0 + 16c + l % 16.
+  //
+  // What the epilogue adds or rotates by: residual rows, or cos and sin of two
+  // pairs, requested with the first chunks (element by element at the end
+  // they cost a round trip each, which a short reduction does not hide).
+  AMMON_DEV void load_pre(f32x4 (&pre)[NT]) const {
+#pragma unroll
+    for (uint32_t c = 0; c < NT; ++c) {
+      pre[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+      const uint32_t t = tok0 + 16 * c + (lane & 15), v = vr0 + 4 * (lane >> 4);
+      if (MODE == AMMON_GEMV_RESIDUAL && t < p.tokens) {
+        const float *at = p.residual + (size_t)t * p.d + v;
+        if (v + 3 < p.d)
+          pre[c] = *(const f32x4a4 *)at;
+        else
+          for (uint32_t r = 0; r < 4; ++r)
+            if (v + r < p.d) pre[c][r] = at[r];
+      }
+      if (MODE == AMMON_GEMV_QKV && t < p.tokens && v < p.d + p.kv_dim) {
+        const uint32_t pos = p.step->position + t, rr = v < p.d ? v : v - p.d;
+        if (pos < p.seq) pre[c] = *(const f32x4a4 *)(p.table + (size_t)pos * p.head + rr % p.head);
+      }
+    }
+  }
+
+  // Rows v..v + 3 of token t of y (those below p.d).
+  AMMON_DEV void store4(uint32_t t, uint32_t v, f32x4 o) const {
+    float *at = p.y + (size_t)t * p.d + v;
+    if (v + 3 < p.d)
+      *(f32x4a4 *)at = o;
+    else
+      for (uint32_t r = 0; r < 4; ++r)
+        if (v + r < p.d) at[r] = o[r];
+  }
+
   // KS = 1: contains barriers (SWIGLU), call uniformly; KS > 1: wave 0 only,
   // with the summed partials.  xs is free by then.
-  AMMON_DEV void epilogue(f32x4 (&acc)[NT], u32x4 *xs) const {
+  AMMON_DEV void epilogue(f32x4 (&acc)[NT], const f32x4 (&pre)[NT], u32x4 *xs) const {
     const uint32_t rq = 4 * (lane >> 4);
     float *ex = (float *)xs;
+    f32x4 up[NT];
     if (MODE == AMMON_GEMV_SWIGLU && KS > 1) {
       // gate rows sit in lanes 0-31, the matching up rows 32 lanes higher
 #pragma unroll
-      for (uint32_t c = 0; c < NT; ++c) {
-        float up[4];
+      for (uint32_t c = 0; c < NT; ++c)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) up[r] = __shfl_xor(acc[c][r], 32);
-        const uint32_t t = tok0 + 16 * c + (lane & 15);
-        if (lane >= 32 || t >= p.tokens) continue;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const uint32_t i = vr0 + rq + r;
-          if (i >= p.d) continue;
-          const float gate = acc[c][r];
-          float v = gate * (1.0f / (1.0f + expf(-gate)));
-          v = v * up[r];
-          p.y[(size_t)t * p.d + i] = v;
-        }
-      }
-      return;
-    }
-    if (MODE == AMMON_GEMV_SWIGLU) {
+        for (int r = 0; r < 4; ++r) up[c][r] = __shfl_xor(acc[c][r], 32);
+      if (lane >= 32) return;
+    } else if (MODE == AMMON_GEMV_SWIGLU) {
       // waves 2-3 hand their up rows to waves 0-1 through LDS, same lane layout
       __syncthreads();
       if (wave >= 2) {
@@ -266,67 +333,31 @@ struct GemmTile {
       }
       __syncthreads();
       if (wave >= 2) return;
+#pragma unroll
+      for (uint32_t c = 0; c < NT; ++c)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) up[c][r] = ex[(((wave * NT + c) * 4) + r) * 64 + lane];
     }
 #pragma unroll
     for (uint32_t c = 0; c < NT; ++c) {
-      const uint32_t t = tok0 + 16 * c + (lane & 15);
+      const uint32_t t = tok0 + 16 * c + (lane & 15), v = vr0 + rq;
+      if (t >= p.tokens) continue;
       if (MODE == AMMON_GEMV_SWIGLU) {
-        if (t >= p.tokens) continue;
+        f32x4 o;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const uint32_t i = vr0 + rq + r;
-          if (i >= p.d) continue;
-          const float gate = acc[c][r], up = ex[(((wave * NT + c) * 4) + r) * 64 + lane];
-          float v = gate * (1.0f / (1.0f + expf(-gate)));
-          v = v * up;
-          p.y[(size_t)t * p.d + i] = v;
+          const float gate = acc[c][r];
+          o[r] = gate * (1.0f / (1.0f + expf(-gate)));
+          o[r] = o[r] * up[c][r];
         }
+        store4(t, v, o);
       } else if (MODE == AMMON_GEMV_QKV) {
-#pragma clang fp contract(off)
-        if (t >= p.tokens) continue;
-        const uint32_t pos = p.step->position + t;
-        const uint32_t kvd = p.kv_dim;
 #pragma unroll
-        for (int r = 0; r < 4; r += 2) {
-          const uint32_t vr = vr0 + rq + r;
-          if (vr >= p.rows) continue;
-          const float a0 = acc[c][r], a1 = acc[c][r + 1];
-          if (pos >= p.seq) {  // out-of-range position: poison q, touch no cache
-            if (vr < p.d) {
-              p.y[(size_t)t * p.d + vr] = __uint_as_float(0x7fc00000u);
-              p.y[(size_t)t * p.d + vr + 1] = __uint_as_float(0x7fc00000u);
-            }
-            continue;
-          }
-          if (vr < p.d + kvd) {
-            const uint32_t rr = vr < p.d ? vr : vr - p.d;
-            const uint32_t hd = rr % p.head;
-            const float *cs = p.table + ((size_t)pos * (p.head / 2) + hd / 2) * 2;
-            const float fcr = cs[0], fci = cs[1];
-            const float o0 = a0 * fcr - a1 * fci;
-            const float o1 = a0 * fci + a1 * fcr;
-            if (vr < p.d) {
-              p.y[(size_t)t * p.d + vr] = o0;
-              p.y[(size_t)t * p.d + vr + 1] = o1;
-            } else {
-              store_pair_out(p.k_cache, p.kv_dtype, ((size_t)(rr / p.head) * p.seq + pos) * p.head + hd,
-                             o0, o1);
-            }
-          } else {
-            const uint32_t rv = vr - p.d - kvd;
-            store_pair_out(p.v_cache, p.kv_dtype,
-                           ((size_t)(rv / p.head) * p.seq + pos) * p.head + rv % p.head, a0, a1);
-          }
-        }
+        for (int r = 0; r < 4; r += 2)
+          if (v + r < p.rows)
+            qkv_store_pair(p, t, v + r, acc[c][r], acc[c][r + 1], pre[c][r], pre[c][r + 1]);
       } else {
-        if (t >= p.tokens) continue;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const uint32_t vr = vr0 + rq + r;
-          if (vr >= p.rows) continue;
-          const size_t at = (size_t)t * p.d + vr;
-          p.y[at] = MODE == AMMON_GEMV_RESIDUAL ? p.residual[at] + acc[c][r] : acc[c][r];
-        }
+        store4(t, v, MODE == AMMON_GEMV_RESIDUAL ? pre[c] + acc[c] : acc[c]);
       }
     }
   }
@@ -354,6 +385,8 @@ AMMON_DEV void gemm(const ammon_k_gemm &p) {
   tile.load_w(0, wa);
   tile.load_w(1, wb);
   tile.load_x(0, xr);
+  f32x4 pre[NT];
+  tile.load_pre(pre);
   // Two W buffers with fixed roles (unrolled); x one chunk ahead.
   for (uint32_t ch = 0; ch < chunks; ch += 2) {
     __syncthreads();  // the previous chunk's operands are consumed
@@ -390,43 +423,7 @@ AMMON_DEV void gemm(const ammon_k_gemm &p) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[c][r] += ex[(((w - 1) * NT + c) * 4 + r) * 64 + lane];
   }
-  tile.epilogue(acc, xs);
-}
-
-// QKV epilogue of virtual rows (v, v + 1) of token t: rotate q and k pairs
-// with the cos/sin table at position step->position + t; q to y, k and raw
-// v rows to the head-major caches (src/kernels.rs:174-226); a position past
-// the cache poisons q and touches no cache.
-AMMON_DEV void qkv_store_pair(const ammon_k_gemm &p, uint32_t t, uint32_t v, float a0, float a1) {
-#pragma clang fp contract(off)
-  const uint32_t pos = p.step->position + t;
-  const uint32_t kvd = p.kv_dim;
-  if (pos >= p.seq) {
-    if (v < p.d) {
-      p.y[(size_t)t * p.d + v] = __uint_as_float(0x7fc00000u);
-      p.y[(size_t)t * p.d + v + 1] = __uint_as_float(0x7fc00000u);
-    }
-    return;
-  }
-  if (v < p.d + kvd) {
-    const uint32_t rr = v < p.d ? v : v - p.d;
-    const uint32_t hd = rr % p.head;
-    const float *cs = p.table + ((size_t)pos * (p.head / 2) + hd / 2) * 2;
-    const float fcr = cs[0], fci = cs[1];
-    const float o0 = a0 * fcr - a1 * fci;
-    const float o1 = a0 * fci + a1 * fcr;
-    if (v < p.d) {
-      p.y[(size_t)t * p.d + v] = o0;
-      p.y[(size_t)t * p.d + v + 1] = o1;
-    } else {
-      store_pair_out(p.k_cache, p.kv_dtype, ((size_t)(rr / p.head) * p.seq + pos) * p.head + hd,
-                     o0, o1);
-    }
-  } else {
-    const uint32_t rv = v - p.d - kvd;
-    store_pair_out(p.v_cache, p.kv_dtype,
-                   ((size_t)(rv / p.head) * p.seq + pos) * p.head + rv % p.head, a0, a1);
-  }
+  tile.epilogue(acc, pre, xs);
 }
 
 // ---- long prompts: register-blocked tiles ----------------------------------
@@ -583,51 +580,86 @@ struct BigTile {
   }
 
   // Lane l holds rows 4(l / 16)..+3 of each tile for token tok0 + 16c + l % 16.
-  AMMON_DEV void epilogue(const f32x4 (&acc)[RT][NT], uint32_t ks) const {
+  // What a store needs from memory (residual, cos / sin) is requested for
+  // several of them first, and rows of four go out as one 16-byte store where
+  // rows come in fours: element by element the loads of a lane waited for each
+  // other (8B shape, 1000 tokens: wo and w2 349 -> 339 us on average; QKV of 131
+  // tokens, whose ranges' sums leave this way: 65 -> 56 us).
+  AMMON_DEV void epilogue(const f32x4 (&acc)[RT][NT], uint32_t ks) {
+    asm volatile("" : "+v"(lane));  // nothing of it is computed before the loop
     const uint32_t rq = 4 * (lane >> 4);
+    if (MODE == AMMON_GEMV_QKV && p.ksplit <= 1) {
+      float cs[RT][NT][4];
 #pragma unroll
-    for (uint32_t c = 0; c < NT; ++c) {
-      const uint32_t t = tok0 + 16 * c + (lane & 15);
-      if (t >= p.tokens) continue;
-      if (MODE != AMMON_GEMV_SWIGLU && p.ksplit > 1) {
-        float *w = p.ws + ((size_t)ks * p.tokens + t) * p.rows;  // this range's partial sums
+      for (uint32_t j = 0; j < RT; ++j)
 #pragma unroll
-        for (uint32_t j = 0; j < RT; ++j)
+        for (uint32_t c = 0; c < NT; ++c) {
+          const uint32_t t = tok0 + 16 * c + (lane & 15), v = vr[j] + rq;
+          const uint32_t rr = v < p.d ? v : v - p.d, pos = p.step->position + t;
+          const bool rot = t < p.tokens && v < p.d + p.kv_dim && pos < p.seq;
+          const float *at = p.table + (rot ? (size_t)pos * p.head + rr % p.head : 0);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const uint32_t v = vr[j] + rq + i;
-            if (v < p.rows) w[v] = acc[j][c][i];
-          }
-      } else if (MODE == AMMON_GEMV_SWIGLU) {
+          for (int i = 0; i < 4; ++i) cs[j][c][i] = at[i];
+        }
 #pragma unroll
-        for (uint32_t j = 0; j < RT / 2; ++j)
+      for (uint32_t j = 0; j < RT; ++j)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const uint32_t h = vr[j] + rq + i;
-            if (h >= p.d) continue;
-            const float gate = acc[j][c][i], up = acc[j + RT / 2][c][i];
-            float v = gate * (1.0f / (1.0f + expf(-gate)));
-            v = v * up;
-            p.y[(size_t)t * p.d + h] = v;
-          }
-      } else if (MODE == AMMON_GEMV_QKV) {
-#pragma unroll
-        for (uint32_t j = 0; j < RT; ++j)
+        for (uint32_t c = 0; c < NT; ++c)
 #pragma unroll
           for (int i = 0; i < 4; i += 2) {
-            const uint32_t v = vr[j] + rq + i;
-            if (v < p.rows) qkv_store_pair(p, t, v, acc[j][c][i], acc[j][c][i + 1]);
+            const uint32_t t = tok0 + 16 * c + (lane & 15), v = vr[j] + rq + i;
+            if (t < p.tokens && v < p.rows)
+              qkv_store_pair(p, t, v, acc[j][c][i], acc[j][c][i + 1], cs[j][c][i], cs[j][c][i + 1]);
           }
-      } else {
+      return;
+    }
+    const bool split = MODE != AMMON_GEMV_SWIGLU && p.ksplit > 1;
+    const uint32_t width = split ? p.rows : p.d, height = min(p.tokens - tok0, TB);
+    float *y = (split ? p.ws + (size_t)ks * p.tokens * p.rows : p.y) + (size_t)tok0 * width;
+    constexpr uint32_t RO = MODE == AMMON_GEMV_SWIGLU ? (RT + 1) / 2 : RT;  // row tiles out
+    auto value = [&](uint32_t j, uint32_t c, int i) {
+      if (MODE != AMMON_GEMV_SWIGLU) return acc[j][c][i];
+      const float gate = acc[j][c][i], up = acc[j + RT / 2][c][i];
+      float v = gate * (1.0f / (1.0f + expf(-gate)));
+      v = v * up;
+      return v;
+    };
+    // buffer accesses: past the last token or row nothing is read or written
+    // (the host keeps TB rows of y below 2 GiB)
+    const bool fours = width % 4 == 0, add = MODE == AMMON_GEMV_RESIDUAL && !split;
+    const __amdgpu_buffer_rsrc_t yr = make_rsrc(y, height * width * 4);
+    const __amdgpu_buffer_rsrc_t rr =
+        make_rsrc(add ? p.residual + (size_t)tok0 * width : y, add ? height * width * 4 : 0);
 #pragma unroll
-        for (uint32_t j = 0; j < RT; ++j)
+    for (uint32_t j = 0; j < RO; ++j) {
+      const uint32_t v0 = vr[j] + rq;
+      f32x4 out[NT];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const uint32_t v = vr[j] + rq + i;
-            if (v >= p.rows) continue;
-            const size_t at = (size_t)t * p.d + v;
-            p.y[at] = MODE == AMMON_GEMV_RESIDUAL ? p.residual[at] + acc[j][c][i] : acc[j][c][i];
-          }
+      for (uint32_t c = 0; c < NT; ++c) {
+        const uint32_t t = 16 * c + (lane & 15), at = (t * width + v0) * 4;
+        out[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (add && fours)
+          out[c] = __builtin_bit_cast(
+              f32x4, __builtin_amdgcn_raw_buffer_load_b128(rr, t < height && v0 < width ? at : AMMON_OOB, 0, 0));
+        else if (add)
+#pragma unroll
+          for (uint32_t i = 0; i < 4; ++i)
+            out[c][i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                rr, t < height && v0 + i < width ? at + 4 * i : AMMON_OOB, 0, 0));
+      }
+#pragma unroll
+      for (uint32_t c = 0; c < NT; ++c) {
+        const uint32_t t = 16 * c + (lane & 15), at = (t * width + v0) * 4;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) out[c][i] = add ? out[c][i] + value(j, c, i) : value(j, c, i);
+        if (fours)
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, out[c]), yr,
+                                                 t < height && v0 < width ? at : AMMON_OOB, 0, 0);
+        else
+#pragma unroll
+          for (uint32_t i = 0; i < 4; ++i)
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(out[c][i]), yr,
+                                                  t < height && v0 + i < width ? at + 4 * i : AMMON_OOB, 0, 0);
       }
     }
   }

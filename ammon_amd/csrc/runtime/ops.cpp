@@ -755,7 +755,8 @@ ammon_status gemm_check_and_launch(ammon_runtime *rt, ammon_stream stream, const
   // 16..512 tokens (e.g. w2 at 512 tokens: 64-row x 64-token tiles split in
   // two 197 us, unsplit 128-row x 64-token tiles 253 us).
   const uint32_t cus = (uint32_t)std::max(rt->info.compute_units, 1);
-  if (a.w_dtype == AMMON_BF16 && rt->gemm_big != 0) {
+  // (64 rows of y stay below 2 GiB: the tiles' stores take 32-bit offsets)
+  if (a.w_dtype == AMMON_BF16 && rt->gemm_big != 0 && a.rows < (1u << 22)) {
     const uint32_t covered = a.mode == AMMON_GEMV_SWIGLU ? a.d : a.rows;
     const uint32_t per4 = a.mode == AMMON_GEMV_SWIGLU ? 128 : 256;  // RT 4: rows per workgroup
     auto wgs = [&](int t64, int rt4) {

@@ -113,6 +113,33 @@ def test_prefill_gemm_split_reduction(rt, d, n, tokens):
              nbytes)
 
 
+# Row tails of one to four rows per lane, first and last tokens of a tile, and y
+# at a 4-byte boundary (a lane's four rows go out as one store): every element
+# right, the ones before and behind y untouched.
+@pytest.mark.parametrize("d,n,tokens,w_dtype", [
+    (1001, 264, 65, BF16), (1002, 264, 64, BF16), (1003, 264, 130, BF16), (1004, 264, 127, BF16),
+    (515, 4104, 33, BF16), (517, 72, 17, BF16), (37, 64, 16, F32), (39, 64, 31, F32),
+    (40, 64, 33, F32),
+])
+def test_prefill_gemm_row_tails(rt, d, n, tokens, w_dtype):
+    wh = oracle.storage(oracle.normal(d * n, 208, std=0.02), w_dtype).reshape(d, n)
+    xh = oracle.normal(tokens * n, 209).reshape(tokens, n)
+    want = np.stack([oracle.gemv(wh, w_dtype, xh[t]) for t in range(tokens)])
+    w, x = up(rt, wh), up(rt, xh)
+    for residual in (False, True):
+        host = np.full(tokens * d + 8, 7.0, np.float32)
+        if residual:
+            host[1:1 + tokens * d] = oracle.normal(tokens * d, 210)
+        y = up(rt, host)
+        at = ctypes.c_void_p(y.ptr + 4)
+        call("ammon_prefill_gemm", rt.handle, None, w, w_dtype, d, n, x, tokens, at,
+             at if residual else None)
+        got = y.download(tokens * d + 8)
+        base = host[1:1 + tokens * d].reshape(tokens, d) if residual else 0
+        assert rel_err(got[1:1 + tokens * d].reshape(tokens, d), base + want) <= RTOL
+        assert got[0] == 7.0 and (got[1 + tokens * d:] == 7.0).all()
+
+
 def test_prefill_gemm_random_shapes(rt):
     """Seeded random shapes through every tile family and the split
     reduction (rows, reduction length and tokens off every tile multiple),
