@@ -428,12 +428,11 @@ AMMON_DEV void gemm(const ammon_k_gemm &p) {
 
 // ---- long prompts: register-blocked tiles ----------------------------------
 // For prompts of 64 tokens and more a workgroup owns 64 tokens (4 column
-// tiles) x 4 waves x RT 16-row tiles per wave.  Every B fragment (x part)
+// tiles; 32 or 16 for shorter ones) x 4 waves x RT 16-row tiles per wave.  Every B fragment (x part)
 // read from LDS feeds RT MFMAs and every A fragment (W) 12, so a wave issues
 // 3 NT RT MFMAs per 32-wide step against 3 NT LDS and RT global 16-byte
 // reads per lane (the 16-row tiles above: 6 MFMAs per 6 LDS reads), and the
-// x chunk is staged once for 64 RT rows.  W streams six steps (three chunks)
-// ahead of use in registers and x two chunks ahead, so a workgroup's chain
+// x chunk is staged once for 64 RT rows.  W streams three chunks ahead of use in registers and x two chunks ahead, so a workgroup's chain
 // of chunks is not paced by memory latency; x is staged in three LDS
 // buffers, one barrier per chunk.  The
 // arithmetic per output is the 16-row tiles' (W x hi, W x mid, W x lo per
@@ -441,7 +440,15 @@ AMMON_DEV void gemm(const ammon_k_gemm &p) {
 // tiles are gate rows, the last RT/2 the same up rows, paired in registers.
 template <int MODE, uint32_t RT, uint32_t NT_>
 struct BigTile {
-  static constexpr uint32_t NT = NT_, TB = 16 * NT, KC = 64, S = KC / 32;
+  static constexpr uint32_t NT = NT_, TB = 16 * NT, KC = NT == 1 ? 128 : 64, S = KC / 32;
+  // Up to 32 tokens the pass is a read of W, so its loads cover whole lines: the
+  // steps of a chunk are requested together, row tile by row tile (128 bytes of
+  // each row, 256 with NT 1).  The SwiGLU block of 17 tokens at 4096 x 14336:
+  // 91 us step by step (64 bytes of 16 rows at a time), 77 so; of 16 tokens 92
+  // with NT 2 step by step, 77 with NT 1 so, 84 with 512 bytes of a row, 91 with
+  // nontemporal loads.  Larger tiles lose with it (QKV of 500 tokens 120 -> 127
+  // us): their requests come back in bursts.
+  static constexpr bool LINES = NT <= 2;
   static constexpr uint32_t RW = 16 * RT;                // virtual rows per wave
   static constexpr uint32_t RBW = RW * AMMON_WAVES;      // virtual rows per workgroup
   static constexpr uint32_t KG = KC / 8;
@@ -460,8 +467,8 @@ struct BigTile {
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     tok0 = tt * TB;
     row_bytes = p.n * 2;
-    kbeg = p.ksplit > 1 ? ks * p.kchunks * KC : 0;
-    kend = p.ksplit > 1 ? min(kbeg + p.kchunks * KC, p.n) : p.n;
+    kbeg = p.ksplit > 1 ? ks * p.kchunks * 64 : 0;
+    kend = p.ksplit > 1 ? min(kbeg + p.kchunks * 64, p.n) : p.n;
     auto rsrc = [&](const void *base, uint32_t first, uint32_t limit) {
       const uint32_t valid = first < limit ? min(16u, limit - first) : 0;
       return make_rsrc((const uint16_t *)base + (size_t)(valid ? first : 0) * p.n,
@@ -499,6 +506,18 @@ struct BigTile {
     for (uint32_t j = 0; j < RT; ++j) a[j] = __builtin_amdgcn_raw_buffer_load_b128(r[j], off, 0, 0);
   }
 
+  // W of a whole chunk, row tile by row tile (LINES).
+  AMMON_DEV void load_wc(uint32_t ch, u32x4 (&a)[S][RT]) const {
+#pragma unroll
+    for (uint32_t j = 0; j < RT; ++j)
+#pragma unroll
+      for (uint32_t s = 0; s < S; ++s) {
+        const uint32_t k = kbeg + 32 * (S * ch + s) + 8 * (lane >> 4);
+        a[s][j] = __builtin_amdgcn_raw_buffer_load_b128(
+            r[j], k < kend ? (lane & 15) * row_bytes + k * 2 : AMMON_OOB, 0, 0);
+      }
+  }
+
   // x unit u (8 consecutive k of one token) of a chunk: the 64 units of
   // each group u / 64 are 8 tokens x the chunk's 8 k groups, so each wave's
   // two 16-byte loads per unit cover 8 rows of x, 256 contiguous bytes each
@@ -508,8 +527,8 @@ struct BigTile {
   AMMON_DEV static void unit(uint32_t u, uint32_t &s, uint32_t &c, uint32_t &l, uint32_t &t,
                              uint32_t &kg) {
     const uint32_t g = u >> 6, ln = u & 63;
-    t = 8 * g + (ln >> 3);
-    kg = ln & 7;
+    t = 8 * (g % (TB / 8)) + (ln >> 3);
+    kg = 8 * (g / (TB / 8)) + (ln & 7);
     s = kg >> 2;
     c = t >> 4;
     l = (t & 15) + 16 * (kg & 3);
@@ -686,30 +705,34 @@ AMMON_DEV void gemm_big(const ammon_k_gemm &p) {
 #pragma unroll
     for (uint32_t c = 0; c < T::NT; ++c) acc[j][c] = f32x4{0.f, 0.f, 0.f, 0.f};
   const uint32_t chunks = (tile.kend - tile.kbeg + T::KC - 1) / T::KC;
-  // rings: W of steps 2ch .. 2ch + 5 (a0..a5), x of chunks ch .. ch + 2
-  // (x0..x2), LDS buffer ch % 3
-  u32x4 a0[RT], a1[RT], a2[RT], a3[RT], a4[RT], a5[RT];
+  // rings: W of chunks ch .. ch + 2, x of chunks ch .. ch + 2 (x0..x2), LDS
+  // buffer ch % 3
+  constexpr uint32_t S = T::S;
+  u32x4 a[3][S][RT];
   u32x4 x0[T::XU][2], x1[T::XU][2], x2[T::XU][2];
+  auto load_chunk = [&](uint32_t ch) {
+    if constexpr (T::LINES) {
+      tile.load_wc(ch, a[ch]);
+      __builtin_amdgcn_sched_barrier(0);
+    } else {
+#pragma unroll
+      for (uint32_t s = 0; s < S; ++s) {
+        tile.load_w(S * ch + s, a[ch][s]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
   // issue order pinned as the loop's (see below)
-  tile.load_w(0, a0);
-  __builtin_amdgcn_sched_barrier(0);
-  tile.load_w(1, a1);
-  __builtin_amdgcn_sched_barrier(0);
+  load_chunk(0);
   tile.load_x(0, x0);
   __builtin_amdgcn_sched_barrier(0);
-  tile.load_w(2, a2);
-  __builtin_amdgcn_sched_barrier(0);
-  tile.load_w(3, a3);
-  __builtin_amdgcn_sched_barrier(0);
+  load_chunk(1);
   tile.load_x(1, x1);
   __builtin_amdgcn_sched_barrier(0);
-  tile.load_w(4, a4);
-  __builtin_amdgcn_sched_barrier(0);
-  tile.load_w(5, a5);
-  __builtin_amdgcn_sched_barrier(0);
+  load_chunk(2);
   // Chunk c: stage its x (loaded two chunks ago) into LDS buffer c % 3,
-  // then request x of chunk c + 2 and, as each step's W is used, the W six
-  // steps on.  Buffer c % 3 was last read for chunk c - 3, which every wave
+  // then request x of chunk c + 2 and, as each step's W is used, the W three
+  // chunks on.  Buffer c % 3 was last read for chunk c - 3, which every wave
   // finished before the barrier of chunk c - 2.  Requests past the end read
   // zero without touching memory; they are issued anyway so that every path
   // into the loop has the same loads in flight in the same order (the
@@ -717,27 +740,27 @@ AMMON_DEV void gemm_big(const ammon_k_gemm &p) {
   // The scheduling barriers pin the issue order of the phases: the memory
   // counters complete in order, so a load moved later would make every
   // older prefetch wait for it.
-#define BIG_CHUNK(C, XS, XC, XN, WA, WB)                 \
-  {                                                      \
-    tile.stage(XC, xs[XS]);                              \
-    __syncthreads();                                     \
-    tile.load_x((C) + 2, XN);                            \
-    __builtin_amdgcn_sched_barrier(0);                   \
-    tile.compute(0, xs[XS], WA, acc);                    \
-    __builtin_amdgcn_sched_barrier(0);                   \
-    tile.load_w(2 * (C) + 6, WA);                        \
-    __builtin_amdgcn_sched_barrier(0);                   \
-    tile.compute(1, xs[XS], WB, acc);                    \
-    __builtin_amdgcn_sched_barrier(0);                   \
-    tile.load_w(2 * (C) + 7, WB);                        \
-    __builtin_amdgcn_sched_barrier(0);                   \
+#define BIG_CHUNK(C, XS, XC, XN)                                           \
+  {                                                                        \
+    tile.stage(XC, xs[XS]);                                                \
+    __syncthreads();                                                       \
+    tile.load_x((C) + 2, XN);                                              \
+    __builtin_amdgcn_sched_barrier(0);                                     \
+    _Pragma("unroll") for (uint32_t s = 0; s < S; ++s) {                   \
+      tile.compute(s, xs[XS], a[XS][s], acc);                              \
+      __builtin_amdgcn_sched_barrier(0);                                   \
+      if constexpr (!T::LINES) tile.load_w(S * ((C) + 3) + s, a[XS][s]);   \
+      __builtin_amdgcn_sched_barrier(0);                                   \
+    }                                                                      \
+    if constexpr (T::LINES) tile.load_wc((C) + 3, a[XS]);                  \
+    __builtin_amdgcn_sched_barrier(0);                                     \
   }
   // Whole rounds of three chunks: one or two chunks past the end multiply
   // zeros (adding nothing), which keeps the loop body free of exits.
   for (uint32_t ch = 0; ch < chunks; ch += 3) {
-    BIG_CHUNK(ch, 0, x0, x2, a0, a1)
-    BIG_CHUNK(ch + 1, 1, x1, x0, a2, a3)
-    BIG_CHUNK(ch + 2, 2, x2, x1, a4, a5)
+    BIG_CHUNK(ch, 0, x0, x2)
+    BIG_CHUNK(ch + 1, 1, x1, x0)
+    BIG_CHUNK(ch + 2, 2, x2, x1)
   }
 #undef BIG_CHUNK
   tile.epilogue(acc, ks);
@@ -783,6 +806,7 @@ GEMM_BIG_MODES(t64_r4, 4, 4, 2)
 GEMM_BIG_MODES(t64_r2, 2, 4, 2)
 GEMM_BIG_MODES(t32_r4, 4, 2, 2)
 GEMM_BIG_MODES(t32_r2, 2, 2, 4)
+GEMM_BIG_MODES(t16_r2, 2, 1, 2)
 
 // y[t][r] = (residual[t][r] +) the split ranges' partial sums added in range
 // order: grid-stride over tokens x d.

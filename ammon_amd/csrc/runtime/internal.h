@@ -57,6 +57,7 @@ struct Kernels {
   hipFunction_t gemm_reduce_qkv = nullptr;  // ... with the QKV epilogue
   // bf16, register-blocked tiles: [64 tokens, 32 tokens][RT 4, RT 2][mode]
   hipFunction_t gemm_big[2][2][kGemvModes] = {};
+  hipFunction_t gemm_big_t16[kGemvModes] = {};  // 16 tokens, RT 2
 };
 
 // LDS per compute unit on gfx950 (bytes); bounds resident GEMV workgroups.

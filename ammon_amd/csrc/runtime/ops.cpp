@@ -743,8 +743,8 @@ ammon_status gemm_check_and_launch(ammon_runtime *rt, ammon_stream stream, const
   p.head = a.head;
   p.seq = a.seq;
   p.kv_dtype = (uint32_t)a.kv_dtype;
-  // bf16 W: register-blocked tiles of 64 or 32 tokens x 4 waves x 4 or 2
-  // 16-row tiles per wave, the reduction optionally split into 2..8 ranges
+  // bf16 W: register-blocked tiles of 64 or 32 tokens (16 for up to 16) x 4
+  // waves x 4 or 2 (2) 16-row tiles per wave, the reduction optionally split into 2..8 ranges
   // (plain / residual with a workspace).  Take the largest tile whose grid,
   // split into ranges of at least 16 chunks, gives at least 3/4 of a
   // workgroup per CU, with the smallest split that does; else (64+ tokens,
@@ -782,7 +782,7 @@ ammon_status gemm_check_and_launch(ammon_runtime *rt, ammon_stream stream, const
     } else {
       const int order[4][2] = {{1, 1}, {1, 0}, {0, 1}, {0, 0}};
       for (const auto &o : order)
-        if ((a.tokens >= 64 || !o[0]) && wgs(o[0], o[1]) * kmax >= need) {
+        if ((a.tokens >= 64 || !o[0]) && (a.tokens > 16 || !o[1]) && wgs(o[0], o[1]) * kmax >= need) {
           t64 = o[0];
           rt4 = o[1];
           break;
@@ -803,7 +803,9 @@ ammon_status gemm_check_and_launch(ammon_runtime *rt, ammon_stream stream, const
         p.kchunks = cdiv(chunks, ksplit);
       }
       AMMON_CHECK(groups * 8 * tiles * ksplit < (1ull << 31), "%s: grid too large", what);
-      ammon_status st = launch(rt, stream, rt->k.gemm_big[t64 ? 0 : 1][rt4 ? 0 : 1][a.mode],
+      hipFunction_t f = a.tokens <= 16 && !t64 && !rt4 ? rt->k.gemm_big_t16[a.mode]
+                                                       : rt->k.gemm_big[t64 ? 0 : 1][rt4 ? 0 : 1][a.mode];
+      ammon_status st = launch(rt, stream, f,
                                (uint32_t)(groups * 8 * tiles * ksplit), 1, 0, p, what);
       if (st != AMMON_OK || ksplit == 1) return st;
       // the ranges' sums (QKV: per row pair, then the rotation and stores)

@@ -172,6 +172,11 @@ static ammon_status load_kernels(ammon_runtime *rt) {
                  r ? 2 : 4);
         R(6, name, k.gemm_big[t][r][m]);
       }
+  for (int m = 0; m < kGemvModes; ++m) {
+    char name[96];
+    snprintf(name, sizeof name, "ammon_gemm_bf16_%s_t16_r2", modes[m]);
+    R(6, name, k.gemm_big_t16[m]);
+  }
 #undef R
   return AMMON_OK;
 }

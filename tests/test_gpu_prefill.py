@@ -120,6 +120,7 @@ def test_prefill_gemm_split_reduction(rt, d, n, tokens):
     (1001, 264, 65, BF16), (1002, 264, 64, BF16), (1003, 264, 130, BF16), (1004, 264, 127, BF16),
     (515, 4104, 33, BF16), (517, 72, 17, BF16), (37, 64, 16, F32), (39, 64, 31, F32),
     (40, 64, 33, F32),
+    (32770, 136, 16, BF16), (24577, 648, 1, BF16),  # 16-token tiles of many rows
 ])
 def test_prefill_gemm_row_tails(rt, d, n, tokens, w_dtype):
     wh = oracle.storage(oracle.normal(d * n, 208, std=0.02), w_dtype).reshape(d, n)
@@ -138,6 +139,23 @@ def test_prefill_gemm_row_tails(rt, d, n, tokens, w_dtype):
         base = host[1:1 + tokens * d].reshape(tokens, d) if residual else 0
         assert rel_err(got[1:1 + tokens * d].reshape(tokens, d), base + want) <= RTOL
         assert got[0] == 7.0 and (got[1 + tokens * d:] == 7.0).all()
+
+
+# 16-token tiles (enough row blocks for the device): first and last tokens, row
+# blocks and 128-wide chunks of k that end early; 17 tokens take the next tile.
+@pytest.mark.parametrize("dim,hidden,tokens", [(200, 12300, 1), (136, 12288, 16), (640, 12289, 9),
+                                               (264, 12300, 17)])
+def test_prefill_gate_up_short(rt, dim, hidden, tokens):
+    w1 = oracle.storage(oracle.normal(hidden * dim, 211, std=0.05), BF16).reshape(hidden, dim)
+    w3 = oracle.storage(oracle.normal(hidden * dim, 212, std=0.05), BF16).reshape(hidden, dim)
+    xh = oracle.normal(tokens * dim, 213).reshape(tokens, dim)
+    hb = rt.alloc(tokens * hidden * 4)
+    call("ammon_prefill_gate_up_swiglu", rt.handle, None, up(rt, xh), tokens, up(rt, w1), up(rt, w3),
+         BF16, dim, hidden, hb)
+    got = hb.download((tokens, hidden))
+    for t in range(tokens):
+        gate, lift = (oracle.gemv(w, BF16, xh[t]).astype(np.float64) for w in (w1, w3))
+        assert rel_err(got[t], gate / (1 + np.exp(-gate)) * lift) <= RTOL
 
 
 def test_prefill_gemm_random_shapes(rt):
