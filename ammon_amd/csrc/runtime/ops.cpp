@@ -674,8 +674,10 @@ ammon_status ammon_attention_prefill(ammon_runtime *rt, ammon_stream stream, con
                     "attention_prefill");
     if (st != AMMON_OK || p.splits == 1) return st;
   } else {
+    // one split: the units write the merge's result themselves, as in decode
+    p.single_out = splits == 1;
     st = launch_att(rt, stream, f, splits, kv_heads, tokens, p, "attention_prefill");
-    if (st != AMMON_OK) return st;
+    if (st != AMMON_OK || splits == 1) return st;
   }
   return launch_att(rt, stream, rt->k.att_combine_waves, cdiv(q_heads, kWaves), 1, tokens, p,
                     "attention_prefill");
