@@ -746,18 +746,24 @@ ammon_status gemm_check_and_launch(ammon_runtime *rt, ammon_stream stream, const
   p.seq = a.seq;
   p.kv_dtype = (uint32_t)a.kv_dtype;
   // bf16 W: register-blocked tiles of 64 or 32 tokens (16 for up to 16) x 4
-  // waves x 4 or 2 (2) 16-row tiles per wave, the reduction optionally split into 2..8 ranges
-  // (plain / residual with a workspace).  Take the largest tile whose grid,
-  // split into ranges of at least 16 chunks, gives at least 3/4 of a
-  // workgroup per CU, with the smallest split that does; else (64+ tokens,
-  // or a splittable reduction) the smallest tile split into ranges of at
-  // least 8 chunks; below 64 tokens a projection that fills the device no
-  // way keeps the 16/32-token tiles below, whose reduction split over the
-  // waves suits few rows.  Measured on the Llama-3-8B projections at
-  // 16..512 tokens (e.g. w2 at 512 tokens: 64-row x 64-token tiles split in
-  // two 197 us, unsplit 128-row x 64-token tiles 253 us).
-  const uint32_t cus = (uint32_t)std::max(rt->info.compute_units, 1);
+  // waves x 4 or 2 (2) 16-row tiles per wave, the reduction optionally split
+  // into 2..8 ranges of at least 8 chunks (plain / residual / QKV with a
+  // workspace).  Of all of them the one with the least estimated time, us:
+  // a workgroup takes 1.5 to start and chunk_us per chunk alone on its CU; two
+  // and more on a CU take turns, share of that each (the CU with one more than
+  // the others is what the launch waits for); a split adds its second launch
+  // and the sums' traffic.  Fitted at 4096 x 4096, 6144 x 4096, 4096 x 14336
+  // and 28672 x 4096 (rows x n) and 20 to 1000 tokens, within 15%; e.g. 6144 x
+  // 4096, 131 tokens: 64 x 4 tiles in four ranges 58 us (288 workgroups, one
+  // or two per CU), 32 x 4 in two 42 us (240).
+  //
+  // Short prompts whose smallest tiles are too few for the device, whole or
+  // split, keep the 16/32-token tiles below, which have more and smaller
+  // workgroups: gate/up of 16 tokens at 2 x 5632 x 2048 18 us (20 in 88 register-
+  // blocked tiles), of 40 tokens at 2 x 2816 x 2048 23 (22 in 88), at 2 x 5632 x
+  // 2048 31 (23 in 176).
   // (64 rows of y stay below 2 GiB: the tiles' stores take 32-bit offsets)
+  const uint32_t cus = (uint32_t)std::max(rt->info.compute_units, 1);
   if (a.w_dtype == AMMON_BF16 && rt->gemm_big != 0 && a.rows < (1u << 22)) {
     const uint32_t covered = a.mode == AMMON_GEMV_SWIGLU ? a.d : a.rows;
     const uint32_t per4 = a.mode == AMMON_GEMV_SWIGLU ? 128 : 256;  // RT 4: rows per workgroup
@@ -766,39 +772,32 @@ ammon_status gemm_check_and_launch(ammon_runtime *rt, ammon_stream stream, const
     };
     const uint32_t chunks = (uint32_t)cdiv(a.n, 64);
     const bool splittable = a.ws && a.mode != AMMON_GEMV_SWIGLU;
-    // the most ranges of at least `len` chunks the workspace holds
-    auto kmax_of = [&](uint32_t len) {
-      uint32_t k = 1;
-      if (splittable)
-        while (k < 8 && chunks / (k * 2) >= len &&
-               (uint64_t)k * 2 * a.tokens * a.rows * 4 <= a.ws_bytes)
-          k *= 2;
-      return k;
-    };
-    uint32_t kmax = kmax_of(16);
-    const uint64_t need = ((uint64_t)cus * 3 + 3) / 4;
     int t64 = -1, rt4 = 0;
-    if (rt->gemm_big > 0) {
-      t64 = rt->gemm_big / 10 == 4;
-      rt4 = rt->gemm_big % 10 == 4;
-    } else {
-      const int order[4][2] = {{1, 1}, {1, 0}, {0, 1}, {0, 0}};
-      for (const auto &o : order)
-        if ((a.tokens >= 64 || !o[0]) && (a.tokens > 16 || !o[1]) && wgs(o[0], o[1]) * kmax >= need) {
-          t64 = o[0];
-          rt4 = o[1];
-          break;
+    uint32_t ksplit = 1;
+    double best = 1e300;
+    const bool any = rt->gemm_big > 0 || a.tokens >= 64 || splittable ||
+                     wgs(0, 0) >= (uint64_t)cus * (a.tokens > 16 ? 7 : 12) / 16;
+    for (int t = 0; any && t < 2; ++t)
+      for (int r = 0; r < 2; ++r) {
+        if (rt->gemm_big > 0 ? rt->gemm_big != (t ? 40 : 20) + (r ? 4 : 2)
+                             : (t && a.tokens <= 32) || (r && a.tokens <= 16))
+          continue;
+        static const double chunk_us[2][2] = {{0.6, 1.0}, {1.06, 1.54}};
+        static const double share[2][2] = {{0.95, 1.0}, {0.85, 0.85}};
+        const uint32_t round = a.tokens <= 16 ? 6 : 3;  // the kernels' rounds of chunks
+        for (uint32_t k = 1; k <= 8; k *= 2) {
+          const uint64_t sums = (uint64_t)k * a.tokens * a.rows * 4;
+          if (k > 1 && !(splittable && chunks / k >= 8 && sums <= a.ws_bytes)) break;
+          const uint32_t turns = cdiv(wgs(t, r) * k, cus);
+          const double wg = cdiv(cdiv(chunks, k), round) * round * chunk_us[t][r];
+          const double us = (turns > 1 ? turns * (wg * share[t][r] + 1.5) : wg + 1.5) +
+                            (k > 1 ? 2.5 + 0.5 * k + (sums + 2.0 * a.tokens * a.rows * 4) / 3e6 : 0);
+          if (us < best) best = us, t64 = t, rt4 = r, ksplit = k;
         }
-      if (t64 < 0 && (a.tokens >= 64 || splittable)) {
-        t64 = rt4 = 0;
-        kmax = kmax_of(8);
       }
-    }
     if (t64 >= 0) {
       const uint64_t tiles = cdiv(a.tokens, t64 ? 64 : 32);
       const uint64_t groups = cdiv(cdiv(covered, rt4 ? per4 : per4 / 2), 8);
-      uint32_t ksplit = 1;
-      while (ksplit < kmax && wgs(t64, rt4) * ksplit < need) ksplit *= 2;
       if (ksplit > 1) {
         p.ws = (float *)a.ws;
         p.ksplit = ksplit;
