@@ -21,23 +21,26 @@ AMMON_DEV void cand_merge(float &v, uint32_t &i, float v2, uint32_t i2) {
   }
 }
 
-// Workgroup reduction of the candidates; sv / si hold AMMON_WG entries of
-// LDS.  Contains barriers: call uniformly.
+// Workgroup reduction of the candidates; sv / si hold AMMON_WAVES entries of
+// LDS.  Within a wave by lane exchange, the waves' through LDS: one barrier (a
+// tree over LDS takes nine).  The order of merging does not matter.  Call
+// uniformly.
 AMMON_DEV void block_cand_reduce(float &v, uint32_t &i, float *sv, uint32_t *si) {
-  sv[threadIdx.x] = v;
-  si[threadIdx.x] = i;
-  __syncthreads();
-  for (uint32_t s = AMMON_WG / 2; s > 0; s >>= 1) {
-    if (threadIdx.x < s) {
-      float a = sv[threadIdx.x];
-      uint32_t ai = si[threadIdx.x];
-      cand_merge(a, ai, sv[threadIdx.x + s], si[threadIdx.x + s]);
-      sv[threadIdx.x] = a;
-      si[threadIdx.x] = ai;
-    }
-    __syncthreads();
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const float v2 = __shfl_xor(v, off, 64);
+    const uint32_t i2 = __shfl_xor(i, off, 64);
+    cand_merge(v, i, v2, i2);
   }
+  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (lane == 0) {
+    sv[wave] = v;
+    si[wave] = i;
+  }
+  __syncthreads();
   v = sv[0];
   i = si[0];
+#pragma unroll
+  for (int w = 1; w < AMMON_WAVES; ++w) cand_merge(v, i, sv[w], si[w]);
 }
 

@@ -505,7 +505,7 @@ struct GemvPass {
       // the workgroup's candidate; x's LDS is free once every wave is done
       __syncthreads();
       float *sv = xs;
-      uint32_t *si = (uint32_t *)(xs + AMMON_WG);
+      uint32_t *si = (uint32_t *)(xs + AMMON_WAVES);
       block_cand_reduce(cand_v, cand_i, sv, si);
       if (threadIdx.x == 0) {
         st_out(p.cand_v + wg, cand_v);
