@@ -56,6 +56,7 @@ class LlamaModel : public AutoregressiveModel {
   void ensure_prefill(uint32_t n);
   const float *rope_table();
   void deposit(uint32_t token, uint32_t pos, ammon_stream stream);
+  void copy_step(ammon_decode_step *slot, uint32_t token, uint32_t pos, ammon_stream stream);
 
   Runtime rt_;
   ammon_llama_config c_;
@@ -73,7 +74,7 @@ class LlamaModel : public AutoregressiveModel {
   std::unique_ptr<Scheme> token_scheme_, decode_scheme_;
   Tensor rope_table_;
   uint32_t decode_prompt_ = 0xffffffffu;
-  ammon_decode_step *pinned_step_ = nullptr;
+  ammon_decode_step *pinned_step_ = nullptr;  // [2]: deposits, the end of a prefill
   float *pinned_logits_ = nullptr;
   std::vector<float> host_logits_;
   // prompt prefill scratch, [capacity, width] rows
@@ -143,7 +144,7 @@ LlamaModel::LlamaModel(const Runtime &rt, const ammon_llama_config &c, const amm
       Shape::vector((uint32_t)(std::max(ammon_argmax_scratch_bytes(c.vocab),
                                         ammon_greedy_lm_head_scratch_bytes(rt.raw())) / 4)),
       DType::F32);
-  check(ammon_alloc_host(rt.raw(), sizeof(ammon_decode_step), (void **)&pinned_step_), "llama");
+  check(ammon_alloc_host(rt.raw(), 2 * sizeof(ammon_decode_step), (void **)&pinned_step_), "llama");
   check(ammon_alloc_host(rt.raw(), sizeof(float) * c.vocab, (void **)&pinned_logits_), "llama");
   host_logits_.resize(c.vocab);
   check(ammon_stream_create(rt.raw(), &stream_), "llama stream");
@@ -186,10 +187,15 @@ void LlamaModel::deposit(uint32_t token, uint32_t pos, ammon_stream stream) {
   // The pinned staging slot is reused per token: wait for the previous
   // deposit on this stream before overwriting it.
   check(ammon_stream_synchronize(rt_.raw(), stream), "deposit");
-  pinned_step_->token = token;
-  pinned_step_->position = pos;
-  check(ammon_memcpy(rt_.raw(), step_.data(), pinned_step_, sizeof(ammon_decode_step),
-                     AMMON_COPY_H2D, stream),
+  copy_step(pinned_step_, token, pos, stream);
+}
+
+void LlamaModel::copy_step(ammon_decode_step *slot, uint32_t token, uint32_t pos,
+                           ammon_stream stream) {
+  slot->token = token;
+  slot->position = pos;
+  check(ammon_memcpy(rt_.raw(), step_.data(), slot, sizeof(ammon_decode_step), AMMON_COPY_H2D,
+                     stream),
         "deposit");
 }
 
@@ -369,13 +375,18 @@ void LlamaModel::prefill(const int32_t *tokens, uint32_t n, uint32_t start, floa
   check(ammon_gemv_rmsnorm(rt, st, x + (size_t)(n - 1) * c_.dim, rms_final_.data(), AMMON_F32,
                            c_.eps, wcls_.data(), wd, c_.vocab, c_.dim, (float *)logits_.data()),
         "prefill lm head");
-  // the DecodeStep a one-by-one pass would leave: the last token at its position
-  deposit((uint32_t)tokens[n - 1], start + n - 1, st);
+  // the DecodeStep a one-by-one pass would leave: the last token at its
+  // position, from a slot of its own (only prefill writes it, and every prefill
+  // waits for its copy), so it is queued behind the layers without waiting for
+  // them
+  copy_step(pinned_step_ + 1, (uint32_t)tokens[n - 1], start + n - 1, st);
   if (logits) {
-    check(ammon_memcpy(rt, logits, logits_.data(), sizeof(float) * c_.vocab, AMMON_COPY_D2H, st),
+    check(ammon_memcpy(rt, pinned_logits_, logits_.data(), sizeof(float) * c_.vocab,
+                       AMMON_COPY_D2H, st),
           "prefill logits");
   }
   check(ammon_stream_synchronize(rt, st), "prefill");
+  if (logits) std::memcpy(logits, pinned_logits_, sizeof(float) * c_.vocab);
 }
 
 GenerateTokenOutput LlamaModel::generate_prefill(const std::vector<int32_t> &prompt,
