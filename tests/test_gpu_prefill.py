@@ -298,6 +298,25 @@ def test_prefill_qkv_positions_past_cache_poison_q(rt):
         np.testing.assert_array_equal(rows[seq:], 0)
 
 
+# ---- rmsnorm rows ---------------------------------------------------------------------------
+# Rows held in registers, at the edges of 1, 2, 4 and 8 quads per lane, the loops
+# beyond, and weights at 2-, 4- and 8-byte boundaries; in place too.
+@pytest.mark.parametrize("dim", [4, 1020, 1024, 1028, 2048, 2052, 4096, 4100, 8192, 8196, 1030])
+@pytest.mark.parametrize("w_dtype,shift", [(F32, 0), (F32, 1), (BF16, 0), (BF16, 1), (BF16, 4)])
+def test_rmsnorm_row_widths(rt, dim, w_dtype, shift):
+    rows = 3
+    xh = oracle.normal(rows * dim, 221).reshape(rows, dim)
+    wh = oracle.storage(oracle.normal(dim + shift, 222) + np.float32(1), w_dtype)
+    x, w, o = up(rt, xh), up(rt, wh), rt.alloc(rows * dim * 4)
+    at = ctypes.c_void_p(w.ptr + shift * wh.itemsize)
+    call("ammon_rmsnorm", rt.handle, None, x, at, w_dtype, o, rows, dim, 1e-5)
+    got = o.download((rows, dim))
+    want = oracle.rmsnorm(xh, wh[shift:], w_dtype)
+    assert rel_err(got, want) <= RTOL
+    call("ammon_rmsnorm", rt.handle, None, x, at, w_dtype, x, rows, dim, 1e-5)
+    np.testing.assert_array_equal(x.download((rows, dim)), got)
+
+
 # ---- attention ------------------------------------------------------------------------------
 @pytest.mark.parametrize("q_heads,kv_heads,head,seq,p0,T,split,kv_dtype", [
     (32, 8, 128, 512, 0, 40, 16, BF16),
