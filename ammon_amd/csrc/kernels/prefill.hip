@@ -449,6 +449,13 @@ struct BigTile {
   // nontemporal loads.  Larger tiles lose with it (QKV of 500 tokens 120 -> 127
   // us): their requests come back in bursts.
   static constexpr bool LINES = NT <= 2;
+  // Three chunks' products are summed by themselves and then added to the total:
+  // an output's rounding error grows with the square root of the number of
+  // additions at its size, n / 192 here and 3 n / 32 when every product goes to
+  // one sum (QKV of 131 tokens, n 4096, against 64 bits: 1.9e-7 of the result; one
+  // sum per range 3.6e-7 in four ranges, 7.0e-7 in one).  The largest tile has no
+  // registers for it.
+  static constexpr bool TOTALS = !(RT == 4 && NT == 4);
   static constexpr uint32_t RW = 16 * RT;                // virtual rows per wave
   static constexpr uint32_t RBW = RW * AMMON_WAVES;      // virtual rows per workgroup
   static constexpr uint32_t KG = KC / 8;
@@ -699,11 +706,11 @@ AMMON_DEV void gemm_big(const ammon_k_gemm &p) {
   const uint32_t per = MODE == AMMON_GEMV_SWIGLU ? T::RBW / 2 : T::RBW;
   if (rb * per >= covered) return;  // padding of the last group (uniform)
   T tile(p, rb, tt, ks);
-  f32x4 acc[RT][T::NT];
+  f32x4 acc[RT][T::NT], total[RT][T::NT];
 #pragma unroll
   for (uint32_t j = 0; j < RT; ++j)
 #pragma unroll
-    for (uint32_t c = 0; c < T::NT; ++c) acc[j][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (uint32_t c = 0; c < T::NT; ++c) acc[j][c] = total[j][c] = f32x4{0.f, 0.f, 0.f, 0.f};
   const uint32_t chunks = (tile.kend - tile.kbeg + T::KC - 1) / T::KC;
   // rings: W of chunks ch .. ch + 2, x of chunks ch .. ch + 2 (x0..x2), LDS
   // buffer ch % 3
@@ -761,8 +768,18 @@ AMMON_DEV void gemm_big(const ammon_k_gemm &p) {
     BIG_CHUNK(ch, 0, x0, x2)
     BIG_CHUNK(ch + 1, 1, x1, x0)
     BIG_CHUNK(ch + 2, 2, x2, x1)
+    if constexpr (T::TOTALS) {
+#pragma unroll
+      for (uint32_t j = 0; j < RT; ++j)
+#pragma unroll
+        for (uint32_t c = 0; c < NT; ++c) {
+          total[j][c] += acc[j][c];
+          acc[j][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
   }
 #undef BIG_CHUNK
+  if constexpr (T::TOTALS) return tile.epilogue(total, ks);
   tile.epilogue(acc, ks);
 }
 

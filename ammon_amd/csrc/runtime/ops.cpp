@@ -757,6 +757,11 @@ ammon_status gemm_check_and_launch(ammon_runtime *rt, ammon_stream stream, const
   // 4096, 131 tokens: 64 x 4 tiles in four ranges 58 us (288 workgroups, one
   // or two per CU), 32 x 4 in two 42 us (240).
   //
+  // The 64 x 4 tile adds every product of its range to one sum, and rounding
+  // errors grow with the length of that: it keeps at least the `ref` ranges
+  // that fill three quarters of the CUs with ranges of 16 chunks and more (8
+  // where none does).
+  //
   // Short prompts whose smallest tiles are too few for the device, whole or
   // split, keep the 16/32-token tiles below, which have more and smaller
   // workgroups: gate/up of 16 tokens at 2 x 5632 x 2048 18 us (20 in 88 register-
@@ -777,6 +782,22 @@ ammon_status gemm_check_and_launch(ammon_runtime *rt, ammon_stream stream, const
     double best = 1e300;
     const bool any = rt->gemm_big > 0 || a.tokens >= 64 || splittable ||
                      wgs(0, 0) >= (uint64_t)cus * (a.tokens > 16 ? 7 : 12) / 16;
+    const uint64_t need = ((uint64_t)cus * 3 + 3) / 4;
+    auto splits_of = [&](uint32_t len) {
+      uint32_t k = 1;
+      while (splittable && k < 8 && chunks / (k * 2) >= len &&
+             (uint64_t)k * 2 * a.tokens * a.rows * 4 <= a.ws_bytes)
+        k *= 2;
+      return k;
+    };
+    uint32_t ref = 0;
+    for (int i = 3; any && i >= 0; --i) {
+      if ((a.tokens < 64 && i >= 2) || wgs(i >> 1, i & 1) * splits_of(16) < need) continue;
+      for (ref = 1; wgs(i >> 1, i & 1) * ref < need;) ref *= 2;
+      break;
+    }
+    if (any && !ref)
+      for (ref = 1; ref < splits_of(8) && wgs(0, 0) * ref < need;) ref *= 2;
     for (int t = 0; any && t < 2; ++t)
       for (int r = 0; r < 2; ++r) {
         if (rt->gemm_big > 0 ? rt->gemm_big != (t ? 40 : 20) + (r ? 4 : 2)
@@ -788,6 +809,7 @@ ammon_status gemm_check_and_launch(ammon_runtime *rt, ammon_stream stream, const
         for (uint32_t k = 1; k <= 8; k *= 2) {
           const uint64_t sums = (uint64_t)k * a.tokens * a.rows * 4;
           if (k > 1 && !(splittable && chunks / k >= 8 && sums <= a.ws_bytes)) break;
+          if (t && r && k < ref) continue;
           const uint32_t turns = cdiv(wgs(t, r) * k, cus);
           const double wg = cdiv(cdiv(chunks, k), round) * round * chunk_us[t][r];
           const double us = (turns > 1 ? turns * (wg * share[t][r] + 1.5) : wg + 1.5) +
