@@ -11,8 +11,16 @@
 // requested at once and x is read once (two passes of a loop: 16 rows of 4096
 // took 4.8 us, 2048 rows 15.0; so 4.8 and 12.9, and the 16-token SwiGLU block
 // that begins with it 88 -> 83).
-// The order of the sum is the loops'.
+// The sum is the loops', operation for operation (square_sum).
 #include "device_common.h"
+
+// ss + the four squares, each with one rounding, in this order.  Written as
+// sums of products the unrolled form below took the first pair as
+// fma(x0, x0, x1 x1), and a row's result depended on its width and on its
+// weights' alignment.
+AMMON_DEV float square_sum(const float4 &v, float ss) {
+  return fmaf(v.w, v.w, fmaf(v.z, v.z, fmaf(v.y, v.y, fmaf(v.x, v.x, ss))));
+}
 
 // Rows of up to 4 R AMMON_WG elements.
 template <int R>
@@ -36,10 +44,7 @@ AMMON_DEV void rmsnorm_registers(const ammon_k_rmsnorm &p, const float *x, float
   float ss = 0.f;
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    ss += v[r].x * v[r].x;
-    ss += v[r].y * v[r].y;
-    ss += v[r].z * v[r].z;
-    ss += v[r].w * v[r].w;
+    ss = square_sum(v[r], ss);
   }
   ss = block_sum(ss, red);
   ss = ss / (float)p.dim;
@@ -73,11 +78,7 @@ extern "C" __global__ __launch_bounds__(AMMON_WG) void ammon_rmsnorm(ammon_k_rms
   float ss = 0.f;
   if (vec) {
     for (uint32_t c = threadIdx.x; c < p.dim / 4; c += AMMON_WG) {
-      float4 v = ((const float4 *)x)[c];
-      ss += v.x * v.x;
-      ss += v.y * v.y;
-      ss += v.z * v.z;
-      ss += v.w * v.w;
+      ss = square_sum(((const float4 *)x)[c], ss);
     }
   } else {
     for (uint32_t j = threadIdx.x; j < p.dim; j += AMMON_WG) ss += x[j] * x[j];

@@ -317,6 +317,23 @@ def test_rmsnorm_row_widths(rt, dim, w_dtype, shift):
     np.testing.assert_array_equal(x.download((rows, dim)), got)
 
 
+# The same row gives the same bits however its weights are aligned: weights one
+# bf16 off an 8-byte boundary take the loop over the row, aligned ones the forms
+# that hold it in registers.
+@pytest.mark.parametrize("dim", [4, 1020, 1024, 1028, 2048, 2052, 4096, 4100, 8192, 8196])
+def test_rmsnorm_does_not_depend_on_alignment(rt, dim):
+    rows = 64
+    x, o = up(rt, oracle.normal(rows * dim, 223)), rt.alloc(rows * dim * 4)
+    w = oracle.storage(oracle.normal(dim, 224) + np.float32(1), BF16)
+    got = []
+    for shift in (0, 1):
+        at = up(rt, np.concatenate([np.zeros(shift, w.dtype), w]))
+        call("ammon_rmsnorm", rt.handle, None, x, ctypes.c_void_p(at.ptr + 2 * shift), BF16, o, rows,
+             dim, 1e-5)
+        got.append(o.download((rows, dim)))
+    np.testing.assert_array_equal(got[0], got[1])
+
+
 # ---- attention ------------------------------------------------------------------------------
 @pytest.mark.parametrize("q_heads,kv_heads,head,seq,p0,T,split,kv_dtype", [
     (32, 8, 128, 512, 0, 40, 16, BF16),
