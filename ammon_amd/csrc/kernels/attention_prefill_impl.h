@@ -26,17 +26,21 @@
 // With one split a workgroup writes the result, otherwise the partial of its
 // range, which ammon_attention_combine_waves merges.
 //
-// fp32 sums are kept in short chains (per 32 or 16 positions, then one addition
-// per output) wherever one unit per token (decode's) had them short: the
-// error against 64 bits is no larger than that unit's.
+// fp32 sums are kept in short chains: 16, 32 or 64 positions' products by
+// themselves, then one addition per output, over splits of at most 2048
+// positions.  So the error against 64 bits is no larger than that of one unit
+// per token (decode's), also at long contexts: 8:1 heads of 128, bf16 cache,
+// 32768 positions, root mean square of the result: 2.52e-6 (unit 2.53e-6; every
+// product of a split of any length in one sum: 3.10e-6); 6:1: 2.43e-7 (2.57e-7;
+// 6.38e-7); fp32 cache, 8:1: 2.45e-7 (2.92e-7; 6.45e-7).
 //
 // What bounds it.  Matrix work: per (row, position) pair 2 of the score
 // products and 3 of the value products, 2.5 times the bf16 minimum, and about
 // as many VALU cycles for the weights and their parts, which the second
 // workgroup of a CU overlaps.  One unit per (token, kv head) fills 4 of 16
 // columns of each tile at 4:1 and reads K and V once per token.  Measured, 32 q
-// / 8 kv heads of 128, bf16 cache: 2048 tokens 858 -> 93 us (369 TFLOP/s of
-// products once each), 301 tokens after 7001 667 -> 101 us; fp32 cache: 1000
+// / 8 kv heads of 128, bf16 cache: 2048 tokens 858 -> 101 us (340 TFLOP/s of
+// products once each), 301 tokens after 7001 667 -> 104 us; fp32 cache: 1000
 // tokens 352 -> 153 us.
 //
 // Rows land in LDS with their 16-byte pieces XOR-swizzled: K piece p of row r
@@ -125,31 +129,41 @@ struct PrefillTile {
     pp[2] = __builtin_convertvector(r1 - __builtin_convertvector(pp[1], f32x8), bf16x8);
   }
 
-  // O += V P of one chunk.
+  // O += V P of one chunk.  32 or 64 positions' products are summed by
+  // themselves, small parts first, and then added to the output once: a sum that
+  // takes every product rounds 12 times per chunk at the output's size.  The
+  // matrix unit's bf16 sums round downwards (measured: 32768 positions of
+  // zero-mean V gave outputs 2e-7 of their size too low), so with q whole, where
+  // that shows, every second sum is taken of -P and subtracted.
   AMMON_DEV void values(const char *vb, const f32x16 (&p)[SB], f32x16 (&o)[DB]) const {
     if constexpr (BF && NQ == 2) {
+      bf16x8 pp[2 * SB][3];
 #pragma unroll
-      for (int kk = 0; kk < 2 * SB; ++kk) {
-        bf16x8 pp[3];
-        parts(p[kk / 2], kk & 1, pp);
-        i16x8 a[DB];
+      for (int kk = 0; kk < 2 * SB; ++kk) parts(p[kk / 2], kk & 1, pp[kk]);
 #pragma unroll
-        for (int db = 0; db < DB; ++db) a[db] = v_frag(vb, kk, db);
+      for (int db = 0; db < DB; ++db) {
+        f32x16 t;
 #pragma unroll
-        for (int q = 0; q < 3; ++q)
+        for (int i = 0; i < 16; ++i) t[i] = 0.f;
+        i16x8 a[2 * SB];
 #pragma unroll
-          for (int db = 0; db < DB; ++db)
-            o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[db]),
-                                                            pp[q], o[db], 0, 0, 0);
+        for (int kk = 0; kk < 2 * SB; ++kk) a[kk] = v_frag(vb, kk, db);
+#pragma unroll
+        for (int q = 2; q >= 0; --q)
+#pragma unroll
+          for (int kk = 0; kk < 2 * SB; ++kk)
+            t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[kk]), pp[kk][q],
+                                                        t, 0, 0, 0);
+        o[db] += t;
+        __builtin_amdgcn_sched_barrier(0);  // no reading ahead: registers
       }
     } else if constexpr (BF) {
-      // 32 positions' sum first, small parts first, then one addition per
-      // output: the sums' rounding is what is left of the error here
 #pragma unroll
       for (int b = 0; b < SB; ++b) {
         bf16x8 pp[2][3];
-        parts(p[b], 0, pp[0]);
-        parts(p[b], 1, pp[1]);
+        const f32x16 pb = b & 1 ? -p[b] : p[b];
+        parts(pb, 0, pp[0]);
+        parts(pb, 1, pp[1]);
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
           f32x16 t;
@@ -162,7 +176,10 @@ struct PrefillTile {
             for (int k = 0; k < 2; ++k)
               t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[k]), pp[k][q],
                                                           t, 0, 0, 0);
-          o[db] += t;
+          if (b & 1)
+            o[db] -= t;
+          else
+            o[db] += t;
         }
         __builtin_amdgcn_sched_barrier(0);  // no reading ahead: registers
       }

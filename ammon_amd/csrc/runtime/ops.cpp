@@ -280,6 +280,9 @@ hipFunction_t attention_kernel(ammon_runtime *rt, ammon_dtype kv_dtype, uint32_t
   return h128 ? rt->k.att_partial_h128_f32[gi] : rt->k.att_partial[dt][ci][gi];
 }
 
+constexpr uint32_t kPrefillMaxSplit = 2048;
+static_assert(kPrefillMaxSplit >= AMMON_ATTENTION_MAX_SPLIT, "the caller's scratch holds the splits");
+
 // Prefill attention: query tiles (attention_prefill_impl.h), or decode's units
 // once per token?
 struct PrefillPlan {
@@ -289,7 +292,10 @@ struct PrefillPlan {
 
 // Tiles need whole 16-byte pieces of cache rows.  Their splits fill two
 // workgroups per CU and no more, are at least 256 positions (a merge costs as
-// much as three chunks) and at most as many as the caller's scratch holds.
+// much as three chunks) and at most as many as the caller's scratch holds.  A
+// split is no longer than kPrefillMaxSplit: its chunks are added to one sum, whose
+// rounding grows with their number (the scratch of a split_len, at most half of
+// that, always holds enough).
 //
 // A tile's time is its serial chain of chunks whatever the number of rows, a
 // unit's is short but there is one per token, so the two are estimated, in
@@ -309,7 +315,8 @@ PrefillPlan prefill_plan(ammon_runtime *rt, uint32_t tokens, uint32_t q_heads, u
   const uint64_t units = (uint64_t)cdiv(rows, 128) * kv_heads;
   const uint64_t slots = 2ull * std::max(rt->info.compute_units, 1);
   const uint64_t want = std::min<uint64_t>(std::max<uint64_t>(slots / units, 1), scratch_splits);
-  const uint32_t split_len = std::max<uint32_t>(cdiv(cdiv(ctx, want), 64) * 64, 256);
+  const uint32_t split_len = std::min(std::max<uint32_t>(cdiv(cdiv(ctx, want), 64) * 64, 256),
+                                      kPrefillMaxSplit);
   const uint32_t splits = cdiv(ctx, split_len);
   if (units * splits >= (1ull << 31)) return plan;
   const bool staged = bf && head == 128 && (g & (g - 1)) == 0;

@@ -424,6 +424,43 @@ def test_attention_prefill_tiles(rt, q_heads, kv_heads, head, kv_dtype, p0, T, s
         assert np.isnan(got[T - 2:]).all()
 
 
+# Long contexts: the tiles' sums (up to 2048 positions each) are no further off
+# than the units', which run the same tokens one by one.  q = 0 makes every weight
+# exactly 1: only the value sums are left to round.  Over 24 tokens x 8 heads x 128
+# outputs the two root mean squares are known within 1 / sqrt(2 x 24576), 0.5%.
+@pytest.mark.parametrize("ctx", [16384, 32768])
+@pytest.mark.parametrize("q_heads,kv_heads,kv_dtype", [(8, 1, BF16), (8, 1, F32), (6, 1, BF16)])
+@pytest.mark.parametrize("q_scale", [0.0, 1.0])
+def test_attention_prefill_long_context_error(rt, q_heads, kv_heads, kv_dtype, ctx, q_scale):
+    head, T, split = 128, 8192, 1024
+    p0 = ctx - T
+    k = oracle.storage(oracle.normal(ctx * head, 264), kv_dtype).reshape(ctx, head)
+    v = oracle.storage(oracle.normal(ctx * head, 265), kv_dtype).reshape(ctx, head)
+    qh = (oracle.normal(T * q_heads * head, 266) * np.float32(q_scale)).reshape(T, q_heads, head)
+    kc, vc, q, out = up(rt, k), up(rt, v), up(rt, qh), rt.alloc(T * q_heads * head * 4)
+    nbytes = _abi.lib.ammon_attention_prefill_scratch_bytes(T, q_heads, head, ctx, split)
+    part = rt.alloc(nbytes)
+
+    def attention(at, tokens, first):
+        call("ammon_attention_prefill", rt.handle, None, at, tokens, q_heads, kc, vc, kv_dtype,
+             kv_heads, head, ctx, rt.step(0, first), first + tokens, split, part, nbytes, out)
+        return out.download((T, q_heads, head))
+
+    kw, vw = (oracle.widen(a, kv_dtype).astype(np.float64) for a in (k, v))
+    tiles = attention(q, T, p0)
+    off = {"tiles": 0.0, "units": 0.0}
+    for t in range(T // 24 - 1, T, T // 24):
+        n = p0 + t + 1
+        s = qh[t].astype(np.float64) @ kw[:n].T / np.sqrt(head)
+        w = np.exp(s - s.max(-1, keepdims=True))
+        want = (w @ vw[:n]) / w.sum(-1, keepdims=True)
+        unit = attention(ctypes.c_void_p(q.ptr + t * q_heads * head * 4), 1, p0 + t)[0]
+        off["tiles"] += np.square(tiles[t] - want).sum() / np.square(want).mean()
+        off["units"] += np.square(unit - want).sum() / np.square(want).mean()
+    print({n: (x / (24 * q_heads * head)) ** 0.5 for n, x in off.items()})
+    assert off["tiles"] <= off["units"] * 1.01 ** 2
+
+
 @pytest.mark.parametrize("kv_dtype", [F32, BF16])
 def test_attention_prefill_positions_past_ctx_are_poisoned(rt, kv_dtype):
     # The grid and the scratch cover ctx positions; the host cannot see
