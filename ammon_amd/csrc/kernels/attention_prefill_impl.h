@@ -39,8 +39,8 @@
 // as many VALU cycles for the weights and their parts, which the second
 // workgroup of a CU overlaps.  One unit per (token, kv head) fills 4 of 16
 // columns of each tile at 4:1 and reads K and V once per token.  Measured, 32 q
-// / 8 kv heads of 128, bf16 cache: 2048 tokens 858 -> 101 us (340 TFLOP/s of
-// products once each), 301 tokens after 7001 667 -> 104 us; fp32 cache: 1000
+// / 8 kv heads of 128, bf16 cache: 2048 tokens 858 -> 100 us (344 TFLOP/s of
+// products once each), 301 tokens after 7001 667 -> 105 us; fp32 cache: 1000
 // tokens 352 -> 153 us.
 //
 // Rows land in LDS with their 16-byte pieces XOR-swizzled: K piece p of row r
@@ -74,6 +74,7 @@ struct PrefillTile {
   static constexpr int QF = BF ? 2 * DB : 4 * DB;    // q fragments: 16 (8) dims each
 
   uint32_t lane, h, wave;
+  uint32_t g;               // kv head
   uint32_t t0, t1;          // this split's positions, up to the tile's last
   uint32_t row;             // this lane's query row
   uint32_t qpos;            // its position
@@ -81,10 +82,37 @@ struct PrefillTile {
   uint32_t head, krow;      // dims, bytes of a cache row
   bool live;                // the wave has rows
   __amdgpu_buffer_rsrc_t kres, vres;
+  bf16x8 qb[BF ? QF : 1][NQ];  // q, the score products' B operand
+  f32x4 qf[BF ? 1 : QF];
+
+  // This lane's row in q and out ([tokens, q heads]; past the last: the last).
+  AMMON_DEV size_t row_at(const ammon_k_attention &p) const {
+    const uint32_t G = p.q_heads / p.kv_heads, r = min(row, p.tokens * G - 1), token = r / G;
+    return (size_t)token * p.q_heads + g * G + (r - token * G);
+  }
+
+  // q fragment kk of a row: dims 16 kk + 8 h..+7 in NQ bf16 parts (fp32:
+  // 8 kk + 4 h..+3); dims past the head are zero.
+  AMMON_DEV void q_frag(const float *q, int kk, bf16x8 (&part)[NQ]) const {
+    const uint32_t d = 16 * kk + 8 * h, at = min(d, head - 8);
+    const float4 a = ld_in4(q + at), b = ld_in4(q + at + 4);
+    f32x8 f = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    if (d >= head) f = f32x8{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+      part[i] = __builtin_convertvector(f, bf16x8);
+      f = f - __builtin_convertvector(part[i], f32x8);
+    }
+  }
+  AMMON_DEV f32x4 q_frag(const float *q, int kk) const {
+    const uint32_t d = 8 * kk + 4 * h;
+    const float4 a = ld_in4(q + min(d, head - 4));
+    return d < head ? f32x4{a.x, a.y, a.z, a.w} : f32x4{0.f, 0.f, 0.f, 0.f};
+  }
 
   // Request chunk c into buffer b: each wave four 1 KiB requests of K, four of
   // V.  Rows at or past t1 read as zero.
-  AMMON_DEV void stage(char *lds, uint32_t c, uint32_t b) const {
+  AMMON_DEV void stage(char *lds, uint32_t c, uint32_t b, uint32_t lane) const {
     const uint32_t s = lane & (SLOTS - 1);
 #pragma unroll
     for (int v = 0; v < 2; ++v)
@@ -200,149 +228,185 @@ struct PrefillTile {
     }
   }
 
-  // A masked weight is 0, and 0 times an infinity or NaN is not: where a chunk
-  // holds positions past some row's own, V of a later token must not reach the
-  // earlier one.  True if the chunk's V has such an element.
-  AMMON_DEV bool values_not_finite(const char *vb) const {
-    uint32_t bad = 0;
-#pragma unroll 2
-    for (uint32_t i = lane; i < HALF / 16; i += 64) {
-      const u32x4 v = ((const u32x4 *)vb)[i];
+  // ---- elements that are not finite ----------------------------------------
+  // The products of a chunk are right for finite K and V only: the parts of q and P
+  // have signs of their own (inf x mid may be -inf), and a masked weight is 0,
+  // which an infinity turns into NaN, so that V of a later token would reach an
+  // earlier one.  Any of it leaves a result that is not finite, so the wave looks
+  // at its results once, at the end, and repeats the split (again() in run) where
+  // one is not.  The second walk keeps weights at or below 1, as the units do,
+  // multiplies zeros in place of such elements and counts them apart: per result, count 1024 for every such element and its sign for
+  // every infinity (x sign of q, x 1 for a weight above 0).  Counts are whole
+  // numbers below 2^24: exact.
+  struct Split {
+    u32x4 finite, count, sign;  // bf16 pairs
+  };
+  AMMON_DEV static Split split(u32x4 v) {
+    Split s;
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        bad |= BF ? ((v[e] & 0x7f807f80u) + 0x00800080u) & 0x80008000u
-                  : ((v[e] & 0x7f800000u) + 0x00800000u) & 0x80000000u;
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t w = v[e];
+      const uint32_t bad = ((w & 0x7f807f80u) + 0x00800080u) & 0x80008000u;
+      const uint32_t nan = (((w & 0x007f007fu) + 0x007f007fu) & 0x00800080u) << 8 & bad;
+      const uint32_t all = (bad >> 15) * 0xffffu, inf = ((bad ^ nan) >> 15) * 0xffffu;
+      s.finite[e] = w & ~all;
+      s.count[e] = all & 0x44804480u;                        // 1024
+      s.sign[e] = inf & ((w & 0x80008000u) | 0x3f803f80u);   // +-1
     }
-    return __any(bad != 0);
+    return s;
+  }
+  AMMON_DEV static void split(float v, float &finite, float &count, float &sign) {
+    const uint32_t u = __float_as_uint(v) & 0x7fffffffu;
+    finite = u >= 0x7f800000u ? 0.f : v;
+    count = u >= 0x7f800000u ? 1024.f : 0.f;
+    sign = u == 0x7f800000u ? copysignf(1.f, v) : 0.f;
+  }
+  // What those elements add to the result they were counted for.
+  AMMON_DEV static float counted(float e) {
+    const float n = rintf(e * (1.f / 1024.f)), d = fmaf(-1024.f, n, e);
+    float r = __uint_as_float(0x7fc00000u);
+    r = d == n ? INFINITY : r;
+    r = d == -n ? -INFINITY : r;
+    return e == 0.f ? 0.f : r;
+  }
+  AMMON_DEV static f32x16 zero16() {
+    f32x16 z;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) z[i] = 0.f;
+    return z;
+  }
+  AMMON_DEV static f32x16 mfma_bf16(u32x4 a, bf16x8 b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), b, c, 0, 0, 0);
   }
 
-  // ... and then the wave's rows are computed one by one from the cache, up to
-  // each row's own position (lane: dims 2 lane and 2 lane + 1).
-  AMMON_DEV void rows_one_by_one(const ammon_k_attention &p, uint32_t g, uint32_t split,
-                                 uint32_t w0) const {
-    const uint32_t G = p.q_heads / p.kv_heads, rows = p.tokens * G, d = 2 * lane;
-    const float scale2 = 1.4426950408889634f / sqrtf((float)head);
-#pragma unroll 1
-    for (uint32_t r = w0; r < min(w0 + 32, rows); ++r) {
-      const uint32_t token = r / G, qh = g * G + (r - token * G);
-      const uint32_t pos = p.step->position + token;
-      const size_t at = (size_t)token * p.q_heads + qh;
-      const bool mine = d < head, ok = pos < p.limit;
-      float q0 = 0.f, q1 = 0.f, m = -INFINITY, l = 0.f, o0 = 0.f, o1 = 0.f;
-      if (mine) q0 = p.q[at * head + d], q1 = p.q[at * head + d + 1];
-#pragma unroll 1
-      for (uint32_t t = t0; ok && t < t1 && t <= pos; ++t) {
-        const size_t k = ((size_t)g * p.seq + t) * head + (mine ? d : 0);
-        const float k0 = load_elem(p.k_cache, DTYPE, k), k1 = load_elem(p.k_cache, DTYPE, k + 1);
-        const float v0 = load_elem(p.v_cache, DTYPE, k), v1 = load_elem(p.v_cache, DTYPE, k + 1);
-        const float s = wave_sum(mine ? q0 * k0 + q1 * k1 : 0.f) * scale2;
-        const float mn = fmaxf(m, s), mu = mn == -INFINITY ? 0.f : mn;
-        const float a = __builtin_amdgcn_exp2f(m - mu), e = __builtin_amdgcn_exp2f(s - mu);
-        l = l * a + e;
-        o0 = o0 * a + e * v0;
-        o1 = o1 * a + e * v1;
-        m = mn;
+  // Scores and values of a chunk that may hold such elements (q is read again:
+  // registers).
+  AMMON_DEV void scores_counted(const ammon_k_attention &p, const char *kb, uint32_t kat,
+                                f32x16 (&s)[SB]) const {
+    size_t at = row_at(p) * head;
+    asm volatile("" : "+v"(at));  // not ahead of the chunk loop: registers
+    const float *q = p.q + at;
+#pragma unroll
+    for (int b = 0; b < SB; ++b) {
+      f32x16 hi = zero16(), rest = zero16(), n = zero16();
+#pragma unroll
+      for (int kk = 0; kk < QF; ++kk) {
+        const char *ka = kb + (kat ^ (kk << 5)) + b * 32 * ROW;
+        if constexpr (BF) {
+          const Split a = split(*(const u32x4 *)ka);
+          bf16x8 qk[NQ];
+          q_frag(q, kk, qk);
+          u32x4 sign = __builtin_bit_cast(u32x4, qk[0]), one;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const uint32_t w = sign[e], set = ((w & 0x7fff7fffu) + 0x7fff7fffu) & 0x80008000u;
+            sign[e] = (set >> 15) * 0xffffu & ((w & 0x80008000u) | 0x3f803f80u);
+            one[e] = 0x3f803f80u;
+          }
+#pragma unroll
+          for (int part = 0; part < NQ; ++part) {
+            f32x16 &acc = part ? rest : hi;
+            acc = mfma_bf16(a.finite, qk[part], acc);
+          }
+          n = mfma_bf16(a.count, __builtin_bit_cast(bf16x8, one), n);
+          n = mfma_bf16(a.sign, __builtin_bit_cast(bf16x8, sign), n);
+        } else {
+          const f32x4 a = *(const f32x4 *)ka, qk = q_frag(q, kk);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            float finite, count, sign;
+            split(a[e], finite, count, sign);
+            f32x16 &acc = kk & 1 ? rest : hi;
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(finite, qk[e], acc, 0, 0, 0);
+            n = __builtin_amdgcn_mfma_f32_32x32x2f32(count, 1.f, n, 0, 0, 0);
+            n = __builtin_amdgcn_mfma_f32_32x32x2f32(
+                sign, qk[e] == 0.f ? 0.f : copysignf(1.f, qk[e]), n, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);  // (registers, here and below)
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
       }
-      if (p.splits == 1) {
-        const float nan = __uint_as_float(0x7fc00000u);
-        if (mine)
-          *(float2 *)(p.out + at * head + d) = ok ? make_float2(o0 / l, o1 / l) : make_float2(nan, nan);
-      } else if (ok && t0 <= pos) {
-        float *w = p.partial + (at * p.splits + split) * (head + 2);
-        if (mine) *(float2 *)(w + d) = make_float2(o0, o1);
-        if (lane == 0) *(float2 *)(w + head) = make_float2(m * 0.6931471805599453f, l);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[b][i] = hi[i] + rest[i] + counted(n[i]);
+    }
+  }
+
+  AMMON_DEV void values_counted(const char *vb, const f32x16 (&p)[SB], uint32_t first, uint32_t lim,
+                                f32x16 (&o)[DB]) const {
+#pragma unroll
+    for (int b = 0; b < SB; ++b) {
+#pragma unroll
+      for (int db = 0; db < DB; ++db) {
+        f32x16 t = zero16(), n = zero16();
+        if constexpr (BF) {
+#pragma unroll
+          for (int k = 0; k < 2; ++k) {
+            const Split a = split(__builtin_bit_cast(u32x4, v_frag(vb, 2 * b + k, db)));
+            bf16x8 pp[3];
+            parts(p[b], k, pp);
+#pragma unroll
+            for (int q = 2; q >= 0; --q) t = mfma_bf16(a.finite, pp[q], t);
+            u32x4 live, above;  // bf16 ones
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const uint32_t i = 8 * k + 2 * e, at = first + 32 * b + 8 * (i >> 2) + 4 * h + (i & 3);
+              live[e] = (at <= lim ? 0x3f80u : 0u) | (at + 1 <= lim ? 0x3f800000u : 0u);
+              above[e] = live[e] & ((p[b][i] > 0.f ? 0xffffu : 0u) | (p[b][i + 1] > 0.f ? 0xffff0000u : 0u));
+            }
+            n = mfma_bf16(a.count, __builtin_bit_cast(bf16x8, live), n);
+            n = mfma_bf16(a.sign, __builtin_bit_cast(bf16x8, above), n);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        } else {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            float finite, count, sign;
+            split(v_elem(vb, i, db), finite, count, sign);
+            const float live = first + 8 * (i >> 2) + 4 * h + (i & 3) <= lim ? 1.f : 0.f;
+            t = __builtin_amdgcn_mfma_f32_32x32x2f32(finite, p[b][i], t, 0, 0, 0);
+            n = __builtin_amdgcn_mfma_f32_32x32x2f32(count, live, n, 0, 0, 0);
+            n = __builtin_amdgcn_mfma_f32_32x32x2f32(sign, p[b][i] > 0.f ? live : 0.f, n, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[db][i] = o[db][i] + t[i] + counted(n[i]);
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
   }
 
-  // Rows [128 tile, +128) of kv head g over split `split`.
-  AMMON_DEV void run(const ammon_k_attention &p, uint32_t g, uint32_t tile, uint32_t split,
-                     char *lds) {
-    lane = threadIdx.x & 63;
-    h = lane >> 5;
-    wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    head = p.head;
-    krow = head * (uint32_t)sizeof(KV);
-    const uint32_t start = p.step->position;
-    const uint32_t G = p.q_heads / p.kv_heads, rows = p.tokens * G;
-    const uint32_t w0 = tile * PF_ROWS + 32 * wave;  // the wave's first row
-    live = w0 < rows;
-    wmin = start + (live ? w0 : rows - 1) / G;
-    wmax = start + min(w0 + 31, rows - 1) / G;
-    row = w0 + (lane & 31);
-    const uint32_t token = min(row, rows - 1) / G;
-    const uint32_t qh = g * G + (min(row, rows - 1) - token * G);
-    qpos = start + token;
-    const uint32_t last = start + min(tile * PF_ROWS + PF_ROWS - 1, rows - 1) / G;
-    t0 = split * p.split_len;
-    t1 = min(min(last + 1, t0 + p.split_len), p.limit);
-    const bool direct = p.splits == 1;
-    float *out = p.out + ((size_t)token * p.q_heads + qh) * head;
-    if (t0 >= t1) {  // no position of this range is live for any row (uniform)
-      return;
-    }
-    kres = make_rsrc((const KV *)p.k_cache + ((size_t)g * p.seq + t0) * head, (t1 - t0) * krow);
-    vres = make_rsrc((const KV *)p.v_cache + ((size_t)g * p.seq + t0) * head, (t1 - t0) * krow);
-
-    // q: B operand, lane = row; fragment kk holds dims 16 kk + 8 h..+7 (fp32:
-    // 8 kk + 4 h..+3); dims past the head are zero
-    const float *qp = p.q + ((size_t)token * p.q_heads + qh) * head;
-    bf16x8 qb[BF ? QF : 1][NQ];
-    f32x4 qf[BF ? 1 : QF];
-    if constexpr (BF) {
-#pragma unroll
-      for (int kk = 0; kk < QF; ++kk) {
-        const uint32_t d = 16 * kk + 8 * h;
-        f32x8 f = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        if (d < head) {
-          const float4 a = ld_in4(qp + d), b = ld_in4(qp + d + 4);
-          f = f32x8{a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-        }
-#pragma unroll
-        for (int part = 0; part < NQ; ++part) {
-          qb[kk][part] = __builtin_convertvector(f, bf16x8);
-          f = f - __builtin_convertvector(qb[kk][part], f32x8);
-        }
-      }
-    } else {
-#pragma unroll
-      for (int kk = 0; kk < QF; ++kk) {
-        const uint32_t d = 8 * kk + 4 * h;
-        qf[kk] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (d < head) {
-          const float4 a = ld_in4(qp + d);
-          qf[kk] = f32x4{a.x, a.y, a.z, a.w};
-        }
-      }
-    }
-    stage(lds, 0, 0);
-
+  // The split's chunks for the wave's rows (go: or only its share of the
+  // staging): m, l and o of each row.  CARE: the second walk, above.
+  template <bool CARE>
+  AMMON_DEV void walk(const ammon_k_attention &p, char *lds, bool go, f32x16 (&o)[DB], float &m,
+                      float &l) const {
     const float scale2 = 1.4426950408889634f / sqrtf((float)head);  // log2(e) / sqrt(head)
-    f32x16 o[DB];
 #pragma unroll
-    for (int db = 0; db < DB; ++db)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) o[db][i] = 0.f;
-    float m = -INFINITY, l = 0.f;  // l: this lane's positions only, summed at the end
+    for (int db = 0; db < DB; ++db) o[db] = zero16();
+    m = -INFINITY, l = 0.f;  // l: this lane's positions only, summed at the end
     const uint32_t lim = min(qpos, t1 - 1);  // last position of this lane's row
-    const uint32_t kat = (lane & 31) * ROW + ((h ^ (lane & (SLOTS - 1) & 31)) << 4);
-
-    bool tainted = false;
+    stage(lds, 0, 0, lane);
     const uint32_t nch = (t1 - t0 + CH - 1) / CH;
     for (uint32_t c = 0; c < nch; ++c) {
       wait_vmcnt<0>();
       __syncthreads();  // chunk c has landed; the other buffer is consumed
-      if (c + 1 < nch) stage(lds, c + 1, (c + 1) & 1);
+      uint32_t ln = lane;
+      if (CARE || (NQ == 3 && DB == 3))  // offsets computed again, not kept: registers
+        asm volatile("" : "+v"(ln));
+      if (c + 1 < nch) stage(lds, c + 1, (c + 1) & 1, ln);
       const uint32_t first = t0 + c * CH;
-      if (!live || first > wmax) continue;  // uniform per wave
+      if (!go || !live || first > wmax) continue;  // uniform per wave
       const char *kb = lds + (c & 1) * 2 * HALF, *vb = kb + HALF;
       f32x16 s[SB], sp[2];  // sp: sums of their own (short chains of fp32 additions)
 #pragma unroll
       for (int b = 0; b < SB; ++b)
 #pragma unroll
         for (int i = 0; i < 16; ++i) s[b][i] = sp[b][i] = 0.f;
+      const uint32_t kat = (ln & 31) * ROW + (((ln >> 5) ^ (ln & (SLOTS - 1) & 31)) << 4);
+      if constexpr (CARE) scores_counted(p, kb, kat, s);
 #pragma unroll
-      for (int kk = 0; kk < QF; ++kk) {
+      for (int kk = 0; kk < (CARE ? 0 : QF); ++kk) {
         if constexpr (BF) {
           bf16x8 a[SB];
 #pragma unroll
@@ -385,7 +449,7 @@ struct PrefillTile {
 #pragma unroll
         for (int i = 0; i < 16; ++i) mc = fmaxf(mc, s[b][i]);
       mc = pair32_max(mc) * scale2;
-      if (__any(mc > m + PF_SLACK)) {
+      if (__any(mc > (CARE ? m : m + PF_SLACK))) {
         const float mn = fmaxf(m, mc);
         const float sc = mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - mn);
 #pragma unroll
@@ -404,16 +468,20 @@ struct PrefillTile {
           ls[i & 3] += s[b][i];
         }
       l += (ls[0] + ls[1]) + (ls[2] + ls[3]);
-      if (masked && values_not_finite(vb)) tainted = true;
-      values(vb, s, o);
+      if constexpr (CARE)
+        values_counted(vb, s, first, lim, o);
+      else
+        values(vb, s, o);
     }
-    if (tainted) {  // uniform per wave
-      rows_one_by_one(p, g, split, w0);
-      return;
-    }
+  }
+
+  // The result or partial of each row.
+  AMMON_DEV void finish(const ammon_k_attention &p, uint32_t split, const f32x16 (&o)[DB], float m,
+                        float l) const {
     l = pair32_sum(l);
-    if (!live || row >= rows) return;
-    if (direct) {
+    if (!live || row >= p.tokens * (p.q_heads / p.kv_heads)) return;
+    if (p.splits == 1) {
+      float *out = p.out + row_at(p) * head;
       const bool ok = qpos < p.limit;
 #pragma unroll
       for (int db = 0; db < DB; ++db)
@@ -430,7 +498,7 @@ struct PrefillTile {
       return;
     }
     if (qpos >= p.limit || t0 > qpos) return;  // dead for this row: the merge skips it
-    float *w = p.partial + ((size_t)token * p.q_heads * p.splits + (size_t)qh * p.splits + split) * (head + 2);
+    float *w = p.partial + (row_at(p) * p.splits + split) * (head + 2);
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -439,5 +507,68 @@ struct PrefillTile {
         if (d < head) *(float2 *)(w + d) = make_float2(o[db][i], o[db][i + 1]);
       }
     if (h == 0) *(float2 *)(w + head) = make_float2(m * 0.6931471805599453f, l);  // natural-log units
+  }
+
+  // Rows [128 tile, +128) of kv head g over split `split`.
+  AMMON_DEV void run(const ammon_k_attention &p, uint32_t g_, uint32_t tile, uint32_t split,
+                     char *lds) {
+    g = g_;
+    wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    head = p.head;
+    krow = head * (uint32_t)sizeof(KV);
+    const uint32_t start = p.step->position;
+    const uint32_t G = p.q_heads / p.kv_heads, rows = p.tokens * G;
+    const uint32_t w0 = tile * PF_ROWS + 32 * wave;  // the wave's first row
+    live = w0 < rows;
+    wmin = start + (live ? w0 : rows - 1) / G;
+    wmax = start + min(w0 + 31, rows - 1) / G;
+    auto lanes = [&] {
+      uint32_t tid = threadIdx.x;
+      asm volatile("" : "+v"(tid));  // computed again, not kept across a walk: registers
+      lane = tid & 63;
+      h = lane >> 5;
+      row = w0 + (lane & 31);
+      qpos = start + min(row, rows - 1) / G;
+    };
+    lanes();
+    const uint32_t last = start + min(tile * PF_ROWS + PF_ROWS - 1, rows - 1) / G;
+    t0 = split * p.split_len;
+    t1 = min(min(last + 1, t0 + p.split_len), p.limit);
+    if (t0 >= t1) {  // no position of this range is live for any row (uniform)
+      return;
+    }
+    kres = make_rsrc((const KV *)p.k_cache + ((size_t)g * p.seq + t0) * head, (t1 - t0) * krow);
+    vres = make_rsrc((const KV *)p.v_cache + ((size_t)g * p.seq + t0) * head, (t1 - t0) * krow);
+
+    const float *q = p.q + row_at(p) * head;
+#pragma unroll
+    for (int kk = 0; kk < QF; ++kk) {
+      if constexpr (BF)
+        q_frag(q, kk, qb[kk]);
+      else
+        qf[kk] = q_frag(q, kk);
+    }
+
+    f32x16 o[DB];
+    float m, l;
+    walk<false>(p, lds, true, o, m, l);
+    lanes();
+    // again? (what decides it: a row whose result is read)
+    float z = l * 0.f;
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) z = fmaf(o[db][i], 0.f, z);
+    const uint64_t off = __ballot(live && row < rows && qpos < p.limit && t0 <= qpos && !(z == 0.f));
+    if (!off) finish(p, split, o, m, l);
+    __syncthreads();  // the ring is consumed
+    if (lane == 0) ((uint32_t *)lds)[wave] = (uint32_t)off | (uint32_t)(off >> 32);
+    __syncthreads();
+    const u32x4 any = *(const u32x4 *)lds;
+    if (!(any[0] | any[1] | any[2] | any[3])) return;  // uniform: every wave stages
+    __syncthreads();
+    walk<true>(p, lds, off != 0, o, m, l);
+    lanes();
+    if (off) finish(p, split, o, m, l);
   }
 };

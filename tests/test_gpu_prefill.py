@@ -421,7 +421,49 @@ def test_attention_prefill_tiles(rt, q_heads, kv_heads, head, kv_dtype, p0, T, s
                 assert rel_err(got[t], want) <= RTOL, t
         assert np.isfinite(got[:first_bad]).all()
         assert np.isnan(got[first_bad:T - 2, :, head - 1]).all()
+        assert (got[first_bad:T - 2, :, 3] == np.inf).all()
         assert np.isnan(got[T - 2:]).all()
+
+
+# K and V that are not finite give what they give the oracle, whichever tile, chunk
+# or split they fall into: an infinite V its infinity in its column (two of both
+# signs NaN), an infinite K a NaN row or a weight of 0, and neither reaches an
+# earlier token or another column.  Column 9 holds 1e36 and the first 64 scores
+# are 0: its sums fit with weights of at most 1, not with weights against 0.
+@pytest.mark.parametrize("q_heads,kv_heads,head,kv_dtype,p0,T,split", [
+    (32, 8, 128, BF16, 0, 333, 1024), (32, 8, 128, BF16, 1100, 130, 64),
+    (24, 8, 128, BF16, 0, 333, 1024), (14, 2, 96, BF16, 300, 300, 64), (15, 5, 64, BF16, 0, 500, 512),
+    (32, 32, 24, BF16, 0, 700, 1024), (16, 16, 128, F32, 0, 900, 1024), (14, 2, 96, F32, 600, 300, 64),
+    (32, 8, 64, F32, 1, 511, 1024), (32, 32, 32, F32, 0, 700, 1024),
+])
+def test_attention_prefill_not_finite(rt, q_heads, kv_heads, head, kv_dtype, p0, T, split):
+    seq = ctx = p0 + T
+    k, v = (oracle.normal(seq * kv_heads * head, s).reshape(seq, kv_heads, head) for s in (267, 268))
+    qh = oracle.normal(T * q_heads * head, 269).reshape(T, q_heads, head)
+    k[:64] = 0
+    v[:, :, 9] = 1e36
+    v[17, :, 3] = v[40, :, 5] = np.inf
+    v[90, :, 5] = -np.inf
+    v[100, :, 7] = np.nan
+    v[p0 + T // 2, :, 1] = -np.inf
+    k[p0 + T // 2 + 2, 0, 4] = np.inf
+    kp, vp = (oracle.storage(a.ravel(), kv_dtype).reshape(seq, kv_heads, head) for a in (k, v))
+    kc, vc = (up(rt, head_major(a, kv_heads, seq, head)) for a in (kp, vp))
+    out = rt.alloc(T * q_heads * head * 4)
+    nbytes = _abi.lib.ammon_attention_prefill_scratch_bytes(T, q_heads, head, ctx, split)
+    call("ammon_attention_prefill", rt.handle, None, up(rt, qh), T, q_heads, kc, vc, kv_dtype,
+         kv_heads, head, seq, rt.step(0, p0), ctx, split, rt.alloc(nbytes), nbytes, out)
+    got = out.download((T, q_heads, head))
+    late = T // 2
+    for t in (0, 1, 16, 17, 39, 40, 41, 63, 64, 90, 101, late - 1, late, late + 1, late + 2, late + 3, T - 1):
+        want = oracle.attention_serial(qh[t], kp, vp, kv_dtype, p0 + t)
+        np.testing.assert_array_equal(np.isnan(got[t]), np.isnan(want), err_msg=str(t))
+        same = np.isinf(want)
+        np.testing.assert_array_equal(got[t][same], want[same], err_msg=str(t))
+        for cols in (np.arange(head) != 9, np.arange(head) == 9):
+            use = np.isfinite(want) & cols
+            if use.any():
+                assert rel_err(got[t][use], want[use]) <= RTOL, t
 
 
 # Long contexts: the tiles' sums (up to 2048 positions each) are no further off
