@@ -85,6 +85,9 @@ typedef struct {
   const void *warm;
   uint32_t warm_row_bytes, warm_rows, warm_bytes, warm_blocks, warm_min_pos;
   uint32_t tokens;          /* prefill tiles: query tokens of the launch */
+  uint32_t pair;            /* prefill tiles: workgroups per XCD of which every CU
+                               gets one, where a second one per CU takes the
+                               rest, in reverse order (0: order as launched) */
 } ammon_k_attention;
 
 typedef struct {

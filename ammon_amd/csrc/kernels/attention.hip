@@ -99,11 +99,12 @@ ATT_KERNEL(ammon_attention_combine_waves) {
 }
 
 // Prefill tiles: one workgroup per (128 query rows, split, kv head), two per CU
-// (registers and LDS allow two).  Unit u = (tile, split, kv head), kv head
-// fastest, tiles from the last (with causal masking the longest) to the first:
-// with 8 kv heads each XCD keeps one head's K and V in its L2.  Workgroups
-// 0..255 land on distinct CUs; where the rest fit beside them they take their
-// units in reverse, so that a CU that runs two gets a long and a short one.
+// (registers and LDS allow two; OCC 1: the registers one).  Unit u = (tile, split,
+// kv head), kv head fastest, tiles from the last (with causal masking the
+// longest) to the first: with 8 kv heads each XCD keeps one head's K and V in its
+// L2.  The first workgroups land on distinct CUs; where the rest fit beside them
+// (p.pair) they take their units in reverse, so that a CU that runs two gets a
+// long and a short one.
 #define ATT_PREFILL(NAME, KV, DB, NQ, OCC)                                                   \
   ATT_KERNEL_OCC(NAME, OCC) {                                                        \
     ATT_PARAMS(p);                                                                   \
@@ -111,7 +112,7 @@ ATT_KERNEL(ammon_attention_combine_waves) {
     const uint32_t rows = p.tokens * (p.q_heads / p.kv_heads);                       \
     const uint32_t tiles = (rows + PF_ROWS - 1) / PF_ROWS;                           \
     const uint32_t b = blockIdx.x >> 3, nb = gridDim.x >> 3;                         \
-    const uint32_t u = (b < 32 || nb > 64 ? b : 32 + nb - 1 - b) * 8 + (blockIdx.x & 7u);       \
+    const uint32_t u = (p.pair && b >= p.pair ? p.pair + nb - 1 - b : b) * 8 + (blockIdx.x & 7u); \
     if (u >= tiles * p.splits * p.kv_heads) return; /* uniform */                    \
     const uint32_t g = u % p.kv_heads, q = u / p.kv_heads;                           \
     PrefillTile<KV, DB, NQ> unit;                                                       \

@@ -287,11 +287,13 @@ static_assert(kPrefillMaxSplit >= AMMON_ATTENTION_MAX_SPLIT, "the caller's scrat
 // once per token?
 struct PrefillPlan {
   hipFunction_t f = nullptr;  // NULL: decode's units
-  uint32_t units = 0, split_len = 0, splits = 0;
+  uint32_t split_len = 0, splits = 0, grid = 0;
+  uint32_t pair = 0;  // ammon_k_attention::pair
 };
 
-// Tiles need whole 16-byte pieces of cache rows.  Their splits fill two
-// workgroups per CU and no more, are at least 256 positions (a merge costs as
+// Tiles need whole 16-byte pieces of cache rows.  Their splits fill the
+// workgroups that are resident at once (two per CU, one of the kernel whose
+// registers allow no more) and no more, are at least 256 positions (a merge costs as
 // much as three chunks) and at most as many as the caller's scratch holds.  A
 // split is no longer than kPrefillMaxSplit: its chunks are added to one sum, whose
 // rounding grows with their number (the scratch of a split_len, at most half of
@@ -313,13 +315,17 @@ PrefillPlan prefill_plan(ammon_runtime *rt, uint32_t tokens, uint32_t q_heads, u
   const uint64_t rows = (uint64_t)tokens * g, krow = head * dsize(kv_dtype);
   if (!aligned || krow % 16 != 0 || ctx * krow >= (1ull << 31) || rows >= (1ull << 31)) return plan;
   const uint64_t units = (uint64_t)cdiv(rows, 128) * kv_heads;
-  const uint64_t slots = 2ull * std::max(rt->info.compute_units, 1);
+  const bool staged = bf && head == 128 && (g & (g - 1)) == 0;
+  hipFunction_t f = staged ? rt->k.att_prefill_h128_bf16 : rt->k.att_prefill[bf ? 1 : 0][(head - 1) / 32];
+  const uint32_t cus = (uint32_t)std::max(rt->info.compute_units, 1);
+  DeviceGuard guard(rt->device);
+  const uint32_t per_cu = occupancy(rt, f, 0);
+  const uint64_t slots = (uint64_t)cus * per_cu;
   const uint64_t want = std::min<uint64_t>(std::max<uint64_t>(slots / units, 1), scratch_splits);
   const uint32_t split_len = std::min(std::max<uint32_t>(cdiv(cdiv(ctx, want), 64) * 64, 256),
                                       kPrefillMaxSplit);
   const uint32_t splits = cdiv(ctx, split_len);
   if (units * splits >= (1ull << 31)) return plan;
-  const bool staged = bf && head == 128 && (g & (g - 1)) == 0;
   const uint32_t db = cdiv(head, 32);
   const double chunk_ns = staged ? 2200 : bf ? 300 + 780 * db : 2000 + 1800 * db;
   const double rounds = std::max(1.0, (double)units * splits / slots);
@@ -333,8 +339,9 @@ PrefillPlan prefill_plan(ammon_runtime *rt, uint32_t tokens, uint32_t q_heads, u
   const double position_ns = staged ? 0.034 : lanes * (head == 128 ? 1.3e-4 * (heads + 1) : 2e-4 * (heads + 0.3));
   const double unit_ns = 8e3 + positions * position_ns;
   if (tile_ns >= unit_ns) return plan;
-  plan.f = staged ? rt->k.att_prefill_h128_bf16 : rt->k.att_prefill[bf ? 1 : 0][(head - 1) / 32];
-  plan.units = (uint32_t)units;
+  plan.f = f;
+  plan.grid = cdiv(units * splits, 8) * 8;
+  if (per_cu >= 2 && cus % 8 == 0 && plan.grid > cus && plan.grid <= 2 * cus) plan.pair = cus / 8;
   plan.split_len = split_len;
   plan.splits = splits;
   return plan;
@@ -486,7 +493,7 @@ ammon_status attention_pass1(ammon_runtime *rt, ammon_stream stream, const float
   const uint32_t splits = ammon_attention_splits(seq, split_len);
   ammon_k_attention p = {q, k_cache, v_cache, (const ammon_k_step *)step, partial, single_out,
                          q_heads, kv_heads, head, seq, split_len, splits, 0, seq,
-                         single_out ? 1u : 0u, nullptr, 0, 0, 0, 0, 0, 1};
+                         single_out ? 1u : 0u, nullptr, 0, 0, 0, 0, 0, 1, 0};
   return launch_att(rt, stream, f, splits, kv_heads, 1, p, "attention_partial");
 }
 }  // namespace
@@ -539,7 +546,7 @@ ammon_status ammon_attention_combine_warm(ammon_runtime *rt, ammon_stream stream
   VALIDATE_ONLY();
   ammon_k_attention p = {nullptr, nullptr, nullptr, (const ammon_k_step *)step, (float *)partial,
                          out, q_heads, 1, head, seq, split_len,
-                         ammon_attention_splits(seq, split_len), 0, seq, 0, nullptr, 0, 0, 0, 0, 0, 1};
+                         ammon_attention_splits(seq, split_len), 0, seq, 0, nullptr, 0, 0, 0, 0, 0, 1, 0};
   const uint32_t grid = q_heads * cdiv(head, 8);
   if (next_w) {
     // The next GEMV (a RESIDUAL-mode ammon_gemv of next_rows x next_n) gives
@@ -670,15 +677,15 @@ ammon_status ammon_attention_prefill(ammon_runtime *rt, ammon_stream stream, con
   const uint32_t splits = ammon_attention_splits(ctx, split_len);
   ammon_k_attention p = {q, k_cache, v_cache, (const ammon_k_step *)step, partial, out,
                          q_heads, kv_heads, head, seq, split_len, splits, 0, ctx, 0, nullptr, 0, 0, 0, 0, 0,
-                         tokens};
+                         tokens, 0};
   const uintptr_t bits = (uintptr_t)q | (uintptr_t)out | (uintptr_t)k_cache | (uintptr_t)v_cache;
   const PrefillPlan plan = prefill_plan(rt, tokens, q_heads, kv_heads, head, ctx, splits, kv_dtype,
                                         (bits & 15u) == 0 && ((uintptr_t)partial & 7u) == 0);
   if (plan.f) {
     p.split_len = plan.split_len;
     p.splits = plan.splits;
-    st = launch_att(rt, stream, plan.f, (plan.units * plan.splits + 7) / 8 * 8, 1, 1, p,
-                    "attention_prefill");
+    p.pair = plan.pair;
+    st = launch_att(rt, stream, plan.f, plan.grid, 1, 1, p, "attention_prefill");
     if (st != AMMON_OK || p.splits == 1) return st;
   } else {
     // one split: the units write the merge's result themselves, as in decode

@@ -425,6 +425,31 @@ def test_attention_prefill_tiles(rt, q_heads, kv_heads, head, kv_dtype, p0, T, s
         assert np.isnan(got[T - 2:]).all()
 
 
+# Splits fill the workgroups that are resident at once: two per CU (the bf16 tile
+# of 4:1 heads of 128), one (3:1, whose q is kept whole).  As many tiles as CUs are
+# split in two in the first case and write their results themselves in the second,
+# leaving the scratch as it was.
+@pytest.mark.parametrize("q_heads,kv_heads,splits", [(32, 8, 2), (24, 8, 1)])
+def test_attention_prefill_splits_follow_residency(rt, q_heads, kv_heads, splits):
+    head, split = 128, 256
+    tiles = rt.info.compute_units // kv_heads
+    T = tiles * 128 // (q_heads // kv_heads)
+    kv = oracle.storage(oracle.normal(2 * T * kv_heads * head, 270), BF16).reshape(2, T, kv_heads, head)
+    qh = oracle.normal(T * q_heads * head, 271).reshape(T, q_heads, head)
+    kc, vc = (up(rt, head_major(a, kv_heads, T, head)) for a in kv)
+    out = rt.alloc(T * q_heads * head * 4)
+    nbytes = _abi.lib.ammon_attention_prefill_scratch_bytes(T, q_heads, head, T, split)
+    part = up(rt, np.full(nbytes // 4, 7.0, np.float32))
+    call("ammon_attention_prefill", rt.handle, None, up(rt, qh), T, q_heads, kc, vc, BF16, kv_heads,
+         head, T, rt.step(0, 0), T, split, part, nbytes, out)
+    got, rest = out.download((T, q_heads, head)), part.download(nbytes // 4)
+    used = T * q_heads * splits * (head + 2) if splits > 1 else 0
+    np.testing.assert_array_equal(rest[used:], 7.0)
+    assert splits == 1 or (rest[:used] != 7.0).any()
+    for t in (0, 1, 127, 128, T // 2, T - 1):
+        assert rel_err(got[t], oracle.attention(qh[t], kv[0], kv[1], BF16, t)) <= RTOL, t
+
+
 # K and V that are not finite give what they give the oracle, whichever tile, chunk
 # or split they fall into: an infinite V its infinity in its column (two of both
 # signs NaN), an infinite K a NaN row or a weight of 0, and neither reaches an
