@@ -877,13 +877,13 @@ AMMON_DEV void attention_combine_wave(const ammon_k_attention &p, uint32_t h) {
 #pragma clang fp contract(off)
   const uint32_t lane = threadIdx.x & 63;
   const uint32_t head = p.head, slot = head + 2;
-  const bool mine = 2 * lane < head;
+  const bool mine = 2 * lane < head, both = 2 * lane + 1 < head;  // (an odd head's last dim)
   float *out = p.out + (size_t)h * head + 2 * lane;
   const uint32_t pos = p.step->position + p.pos_add;
   if (pos >= p.limit) {
     if (mine) {
       st_out(out, __uint_as_float(0x7fc00000u));
-      st_out(out + 1, __uint_as_float(0x7fc00000u));
+      if (both) st_out(out + 1, __uint_as_float(0x7fc00000u));
     }
     return;
   }
@@ -938,6 +938,6 @@ AMMON_DEV void attention_combine_wave(const ammon_k_attention &p, uint32_t h) {
   }
   if (mine) {
     st_out(out, t0 / L);
-    st_out(out + 1, t1 / L);
+    if (both) st_out(out + 1, t1 / L);
   }
 }

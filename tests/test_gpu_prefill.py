@@ -425,6 +425,27 @@ def test_attention_prefill_tiles(rt, q_heads, kv_heads, head, kv_dtype, p0, T, s
         assert np.isnan(got[T - 2:]).all()
 
 
+# Odd heads: the merge writes every dim once, nothing into the next head and nothing
+# behind the last one; positions past ctx too.
+@pytest.mark.parametrize("head", [1, 5, 63])
+def test_attention_prefill_odd_heads(rt, head):
+    q_heads, kv_heads, T, p0, split = 4, 2, 9, 30, 16
+    seq, ctx = p0 + T, p0 + T - 1
+    kv = oracle.normal(2 * seq * kv_heads * head, 272).reshape(2, seq, kv_heads, head)
+    qh = oracle.normal(T * q_heads * head, 273).reshape(T, q_heads, head)
+    kc, vc = (up(rt, head_major(a, kv_heads, seq, head)) for a in kv)
+    out = up(rt, np.full(T * q_heads * head + 4, 7.0, np.float32))
+    nbytes = _abi.lib.ammon_attention_prefill_scratch_bytes(T, q_heads, head, ctx, split)
+    call("ammon_attention_prefill", rt.handle, None, up(rt, qh), T, q_heads, kc, vc, F32, kv_heads, head,
+         seq, rt.step(0, p0), ctx, split, rt.alloc(nbytes), nbytes, out)
+    got = out.download(T * q_heads * head + 4)
+    assert (got[T * q_heads * head:] == 7.0).all()
+    got = got[:T * q_heads * head].reshape(T, q_heads, head)
+    for t in range(T - 1):
+        assert rel_err(got[t], oracle.attention(qh[t], kv[0], kv[1], F32, p0 + t)) <= RTOL, t
+    assert np.isnan(got[T - 1]).all()
+
+
 # Splits fill the workgroups that are resident at once: two per CU (the bf16 tile
 # of 4:1 heads of 128), one (3:1, whose q is kept whole).  As many tiles as CUs are
 # split in two in the first case and write their results themselves in the second,
