@@ -425,6 +425,40 @@ def test_attention_prefill_tiles(rt, q_heads, kv_heads, head, kv_dtype, p0, T, s
         assert np.isnan(got[T - 2:]).all()
 
 
+# Every token and head of the tiles against 64 bits; and tiles they are: q at a
+# 4-byte boundary takes the units, whose results are other bits.
+@pytest.mark.parametrize("q_heads,kv_heads,head,kv_dtype,p0,T,split", TILE_SHAPES + [
+    (32, 8, 128, BF16, 0, 700, 1024), (24, 8, 128, BF16, 0, 333, 1024), (32, 8, 16, F32, 0, 1600, 1024),
+    (32, 32, 32, F32, 0, 700, 1024), (32, 8, 32, F32, 400, 300, 256), (16, 16, 128, BF16, 5, 450, 1024),
+    (24, 6, 48, F32, 0, 1000, 1024), (16, 16, 16, BF16, 0, 900, 1024),
+])
+def test_attention_prefill_every_token(rt, q_heads, kv_heads, head, kv_dtype, p0, T, split):
+    ctx = p0 + T
+    kv = oracle.storage(oracle.normal(2 * ctx * kv_heads * head, 274), kv_dtype).reshape(
+        2, ctx, kv_heads, head)
+    qh = oracle.normal(T * q_heads * head, 275)
+    kc, vc = (up(rt, head_major(a, kv_heads, ctx, head)) for a in kv)
+    nbytes = _abi.lib.ammon_attention_prefill_scratch_bytes(T, q_heads, head, ctx, split)
+    out, part, got = rt.alloc(T * q_heads * head * 4), rt.alloc(nbytes), []
+    for shift in (0, 1):
+        q = up(rt, np.concatenate([np.zeros(shift, np.float32), qh]))
+        call("ammon_attention_prefill", rt.handle, None, ctypes.c_void_p(q.ptr + 4 * shift), T, q_heads,
+             kc, vc, kv_dtype, kv_heads, head, ctx, rt.step(0, p0), ctx, split, part, nbytes, out)
+        got.append(out.download((T, q_heads, head)))
+    assert (got[0] != got[1]).any()
+    k, v = (oracle.widen(a, kv_dtype).astype(np.float64) for a in kv)
+    qh, want = qh.astype(np.float64).reshape(T, q_heads, head), np.empty((T, q_heads, head))
+    late = np.arange(ctx)[None] > p0 + np.arange(T)[:, None]
+    for h in range(q_heads):
+        g = h // (q_heads // kv_heads)
+        s = np.where(late, -np.inf, qh[:, h] @ k[:, g].T / np.sqrt(head))
+        w = np.exp(s - s.max(-1, keepdims=True))
+        want[:, h] = (w @ v[:, g]) / w.sum(-1, keepdims=True)
+    for t in range(T):
+        assert rel_err(got[0][t], want[t]) <= RTOL, t
+        assert rel_err(got[1][t], want[t]) <= RTOL, t
+
+
 # Odd heads: the merge writes every dim once, nothing into the next head and nothing
 # behind the last one; positions past ctx too.
 @pytest.mark.parametrize("head", [1, 5, 63])
@@ -501,7 +535,8 @@ def test_attention_prefill_not_finite(rt, q_heads, kv_heads, head, kv_dtype, p0,
          kv_heads, head, seq, rt.step(0, p0), ctx, split, rt.alloc(nbytes), nbytes, out)
     got = out.download((T, q_heads, head))
     late = T // 2
-    for t in (0, 1, 16, 17, 39, 40, 41, 63, 64, 90, 101, late - 1, late, late + 1, late + 2, late + 3, T - 1):
+    edges = {0, 1, 16, 17, 39, 40, 41, 63, 64, 90, 101, late - 1, late, late + 1, late + 2, late + 3, T - 1}
+    for t in sorted(edges | set(range(0, T, 13))):
         want = oracle.attention_serial(qh[t], kp, vp, kv_dtype, p0 + t)
         np.testing.assert_array_equal(np.isnan(got[t]), np.isnan(want), err_msg=str(t))
         same = np.isinf(want)
