@@ -427,16 +427,16 @@ AMMON_DEV void gemm(const ammon_k_gemm &p) {
 }
 
 // ---- long prompts: register-blocked tiles ----------------------------------
-// For prompts of 64 tokens and more a workgroup owns 64 tokens (4 column
-// tiles; 32 or 16 for shorter ones) x 4 waves x RT 16-row tiles per wave.  Every B fragment (x part)
-// read from LDS feeds RT MFMAs and every A fragment (W) 12, so a wave issues
-// 3 NT RT MFMAs per 32-wide step against 3 NT LDS and RT global 16-byte
-// reads per lane (the 16-row tiles above: 6 MFMAs per 6 LDS reads), and the
-// x chunk is staged once for 64 RT rows.  W streams three chunks ahead of use in registers and x two chunks ahead, so a workgroup's chain
-// of chunks is not paced by memory latency; x is staged in three LDS
-// buffers, one barrier per chunk.  The
-// arithmetic per output is the 16-row tiles' (W x hi, W x mid, W x lo per
-// step, fp32 accumulation) in the same order.  SWIGLU: a wave's first RT/2
+// For prompts of 64 tokens and more a workgroup owns 64 tokens (4 column tiles;
+// 32 or 16 for shorter ones) x 4 waves x RT 16-row tiles per wave.  Every B
+// fragment (x part) read from LDS feeds RT MFMAs and every A fragment (W) 12, so a
+// wave issues 3 NT RT MFMAs per 32-wide step against 3 NT LDS and RT global
+// 16-byte reads per lane (the 16-row tiles above: 6 MFMAs per 6 LDS reads), and
+// the x chunk is staged once for 64 RT rows.  W streams three chunks ahead of use
+// in registers and x two chunks ahead, so a workgroup's chain of chunks is not
+// paced by memory latency; x is staged in three LDS buffers, one barrier per
+// chunk.  The arithmetic per output is the 16-row tiles' (W x hi, W x mid, W x lo
+// per step, fp32 accumulation) in the same order.  SWIGLU: a wave's first RT/2
 // tiles are gate rows, the last RT/2 the same up rows, paired in registers.
 template <int MODE, uint32_t RT, uint32_t NT_>
 struct BigTile {

@@ -214,7 +214,7 @@ ammon_status gemv_check_and_launch(ammon_runtime *rt, ammon_stream stream, const
   const int dt = a.w_dtype == AMMON_BF16 ? 1 : 0;
   size_t lds = shmem;
   // PLAIN_ARGMAX reduces the workgroup's candidates in x's LDS
-  if (a.mode == AMMON_GEMV_PLAIN_ARGMAX) lds = std::max<size_t>(lds, 2 * kWorkgroup * 4);
+  if (a.mode == AMMON_GEMV_PLAIN_ARGMAX) lds = std::max<size_t>(lds, 2 * kWaves * 4);
   hipFunction_t fn = gemv_wide(a, vec)                  ? rt->k.gemv_wide[a.mode == AMMON_GEMV_PLAIN_ARGMAX]
                      : a.mode == AMMON_GEMV_PLAIN_ARGMAX ? rt->k.gemv_argmax[dt][vec]
                                                          : rt->k.gemv[dt][vec][a.mode];
@@ -766,10 +766,13 @@ ammon_status gemm_check_and_launch(ammon_runtime *rt, ammon_stream stream, const
   // a workgroup takes 1.5 to start and chunk_us per chunk alone on its CU; two
   // and more on a CU take turns, share of that each (the CU with one more than
   // the others is what the launch waits for); a split adds its second launch
-  // and the sums' traffic.  Fitted at 4096 x 4096, 6144 x 4096, 4096 x 14336
-  // and 28672 x 4096 (rows x n) and 20 to 1000 tokens, within 15%; e.g. 6144 x
-  // 4096, 131 tokens: 64 x 4 tiles in four ranges 58 us (288 workgroups, one
-  // or two per CU), 32 x 4 in two 42 us (240).
+  // and the sums' traffic.  Checked at 4096 x 4096, 6144 x 4096, 4096 x 14336
+  // and 28672 x 4096 (rows x n) and 20 to 1000 tokens, every tile and split: what
+  // it takes is estimated within 20% and at most 14% slower than the best
+  // (6144 x 4096, 500 tokens: 114 us, 64 x 2 tiles 100), 6% in 46 of 48.  E.g.
+  // 6144 x 4096, 131 tokens: 32 x 2 tiles, whole, 45 us (estimate 41, 240
+  // workgroups), 32 x 4 in two ranges 46 (42), 64 x 4 in four 63 (61, 288
+  // workgroups, one or two per CU).
   //
   // The 64 x 4 tile adds every product of its range to one sum, and rounding
   // errors grow with the length of that: it keeps at least the `ref` ranges
