@@ -39,7 +39,7 @@
 // as many VALU cycles for the weights and their parts, which the second
 // workgroup of a CU overlaps.  One unit per (token, kv head) fills 4 of 16
 // columns of each tile at 4:1 and reads K and V once per token.  Measured, 32 q
-// / 8 kv heads of 128, bf16 cache: 2048 tokens 858 -> 100 us (344 TFLOP/s of
+// / 8 kv heads of 128, bf16 cache: 2048 tokens 858 -> 97 us (354 TFLOP/s of
 // products once each), 301 tokens after 7001 667 -> 105 us; fp32 cache: 1000
 // tokens 352 -> 153 us.
 //
@@ -147,14 +147,29 @@ struct PrefillTile {
     return *(const float *)(vb + at + (8 * (i >> 2) + (i & 3)) * ROW);
   }
 
+  // Two floats as bf16, and what they leave.  (Pair by pair: from eight at a time
+  // the compiler rounded every element a second time to widen it, 64 instructions
+  // a chunk.)
+  AMMON_DEV static uint32_t part2(float &a, float &b) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
+    a -= bf16_lo(w);
+    b -= bf16_hi(w);
+    return w;
+  }
+
   // The eight weights of 16 positions as bf16 parts that sum to them.
   AMMON_DEV static void parts(const f32x16 &p, int kk, bf16x8 (&pp)[3]) {
-    const f32x8 f = kk ? __builtin_shufflevector(p, p, 8, 9, 10, 11, 12, 13, 14, 15)
-                       : __builtin_shufflevector(p, p, 0, 1, 2, 3, 4, 5, 6, 7);
-    pp[0] = __builtin_convertvector(f, bf16x8);
-    const f32x8 r1 = f - __builtin_convertvector(pp[0], f32x8);
-    pp[1] = __builtin_convertvector(r1, bf16x8);
-    pp[2] = __builtin_convertvector(r1 - __builtin_convertvector(pp[1], f32x8), bf16x8);
+    u32x4 w[3];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float a = p[8 * kk + 2 * e], b = p[8 * kk + 2 * e + 1];
+#pragma unroll
+      for (int q = 0; q < 3; ++q) w[q][e] = part2(a, b);
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q) pp[q] = __builtin_bit_cast(bf16x8, w[q]);
   }
 
   // O += V P of one chunk.  32 or 64 positions' products are summed by
@@ -169,20 +184,23 @@ struct PrefillTile {
 #pragma unroll
       for (int kk = 0; kk < 2 * SB; ++kk) parts(p[kk / 2], kk & 1, pp[kk]);
 #pragma unroll
-      for (int db = 0; db < DB; ++db) {
-        f32x16 t;
+      for (int db = 0; db < DB; db += 2) {
+        // two chains in turn (one block of dims at a time: 2048 tokens 97 -> 99 us)
+        f32x16 t[2];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) t[i] = 0.f;
-        i16x8 a[2 * SB];
+        for (int i = 0; i < 16; ++i) t[0][i] = t[1][i] = 0.f;
 #pragma unroll
-        for (int kk = 0; kk < 2 * SB; ++kk) a[kk] = v_frag(vb, kk, db);
+        for (int kk = 0; kk < 2 * SB; ++kk) {
+          const i16x8 a[2] = {v_frag(vb, kk, db), v_frag(vb, kk, db + 1)};
 #pragma unroll
-        for (int q = 2; q >= 0; --q)
+          for (int q = 2; q >= 0; --q)
 #pragma unroll
-          for (int kk = 0; kk < 2 * SB; ++kk)
-            t = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[kk]), pp[kk][q],
-                                                        t, 0, 0, 0);
-        o[db] += t;
+            for (int e = 0; e < 2; ++e)
+              t[e] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[e]),
+                                                             pp[kk][q], t[e], 0, 0, 0);
+        }
+        o[db] += t[0];
+        o[db + 1] += t[1];
         __builtin_amdgcn_sched_barrier(0);  // no reading ahead: registers
       }
     } else if constexpr (BF) {
