@@ -316,6 +316,16 @@ PrefillPlan prefill_plan(ammon_runtime *rt, uint32_t tokens, uint32_t q_heads, u
   if (!aligned || krow % 16 != 0 || ctx * krow >= (1ull << 31) || rows >= (1ull << 31)) return plan;
   const uint64_t units = (uint64_t)cdiv(rows, 128) * kv_heads;
   const bool staged = bf && head == 128 && (g & (g - 1)) == 0;
+  const uint32_t db = cdiv(head, 32);
+  const double chunk_ns = staged ? 2200 : bf ? 300 + 780 * db : 2000 + 1800 * db;
+  // a VALU unit's lanes cover the head and its heads the group in powers of two
+  uint32_t lanes = 2, heads = 1;
+  while (lanes < head) lanes <<= 1;
+  while (heads < g) heads <<= 1;
+  const double positions = (double)tokens * kv_heads * (ctx - tokens / 2.0);
+  const double position_ns = staged ? 0.034 : lanes * (head == 128 ? 1.3e-4 * (heads + 1) : 2e-4 * (heads + 0.3));
+  const double unit_ns = 8e3 + positions * position_ns;
+  if (9e3 + chunk_ns >= unit_ns) return plan;  // (the shortest tiles: a small call asks no further)
   hipFunction_t f = staged ? rt->k.att_prefill_h128_bf16 : rt->k.att_prefill[bf ? 1 : 0][(head - 1) / 32];
   const uint32_t cus = (uint32_t)std::max(rt->info.compute_units, 1);
   DeviceGuard guard(rt->device);
@@ -326,18 +336,9 @@ PrefillPlan prefill_plan(ammon_runtime *rt, uint32_t tokens, uint32_t q_heads, u
                                       kPrefillMaxSplit);
   const uint32_t splits = cdiv(ctx, split_len);
   if (units * splits >= (1ull << 31)) return plan;
-  const uint32_t db = cdiv(head, 32);
-  const double chunk_ns = staged ? 2200 : bf ? 300 + 780 * db : 2000 + 1800 * db;
   const double rounds = std::max(1.0, (double)units * splits / slots);
   const double tile_ns = 9e3 + chunk_ns * cdiv(std::min(split_len, ctx), 64) * rounds +
                          (splits > 1 ? 8e3 : 0);
-  // a VALU unit's lanes cover the head and its heads the group in powers of two
-  uint32_t lanes = 2, heads = 1;
-  while (lanes < head) lanes <<= 1;
-  while (heads < g) heads <<= 1;
-  const double positions = (double)tokens * kv_heads * (ctx - tokens / 2.0);
-  const double position_ns = staged ? 0.034 : lanes * (head == 128 ? 1.3e-4 * (heads + 1) : 2e-4 * (heads + 0.3));
-  const double unit_ns = 8e3 + positions * position_ns;
   if (tile_ns >= unit_ns) return plan;
   plan.f = f;
   plan.grid = cdiv(units * splits, 8) * 8;
